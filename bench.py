@@ -223,10 +223,11 @@ def main():
                  "bf16": "k_gvf_sr2<BF16, BF16, BF16, false>"}[args.storage]
         bytes_per_voxel = 18  # v and f read, v written: 3 components x 2 bytes each
     else:
-        spl = args.fuse
+        # F32 runs group iterations as is fastest (four a launch at this size)
+        spl = 4 if args.storage == "f32" and args.fuse >= 2 else args.fuse
         K = 48 // spl
         launch_ms = (gvf_time(spl * (K + 2)) - gvf_time(2 * spl)) / K
-        gk = {4: "k_gvf_fused4<{}, false>", 2: "k_gvf_fused2<{}, false>"}.get(spl, "k_gvf_march<{}, 2, false>")
+        gk = {4: "k_gvf_cols<{}, 4>", 2: "k_gvf_cols<{}, 2>"}.get(spl, "k_gvf_march<{}, 2, false>")
         kname = gk.format(args.storage.upper())
         bytes_per_voxel = 9 * (4 if S == tsf.STORAGE_F32 else 2)
     achieved = bytes_per_voxel * N / (launch_ms * 1e-3)

@@ -4,6 +4,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
+
 #include "tsf_common.hpp"
 
 namespace tsf {
@@ -53,6 +55,18 @@ tsf_status check_field(const tsf_field* f, bool need_w, const char* what) {
 }
 
 size_t storage_bytes(int storage) { return storage == TSF_STORAGE_F32 ? 4 : 2; }
+
+int cu_count() {
+    static std::atomic<int> known[64];  // 0: not asked yet
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = known[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        known[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
 
 Scratch::~Scratch() {
     if (owned && ptr) (void)hipFree(ptr);

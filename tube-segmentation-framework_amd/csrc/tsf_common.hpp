@@ -151,6 +151,7 @@ tsf_status check_launch(const char* what);
 tsf_status check_dims(tsf_dims d, int min_extent, const char* what);
 tsf_status check_field(const tsf_field* f, bool need_w, const char* what);
 size_t storage_bytes(int storage);
+int cu_count();  // compute units of the current device
 
 inline Dims D(tsf_dims d) { return Dims{d.x, d.y, d.z}; }
 
