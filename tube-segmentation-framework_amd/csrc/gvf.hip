@@ -291,13 +291,6 @@ static bool cols_ok(float scale_f, float scale_v, Dims d, int steps) {
 // The built forms of k_gvf_cols.  Small tiles keep a small volume's steps
 // short and its workgroups many; four steps per launch save HBM traffic, and
 // three rows per thread the tile's overlap, where a volume fills the chip.
-// occ: workgroups a CU holds; one, full: microseconds per step of one
-// workgroup alone on a CU and of occ of them sharing it (measured at 2 to 136
-// steps per launch, 64^3 to 512^3).
-struct ColsForm {
-    int K, R, NW, occ;
-    float one, full;
-};
 enum { K2_SMALL, K2_TALL, K2_ROWS2, K3, K4_TALL, K4_ROWS3, COLS_FORMS };
 static const ColsForm FORMS_F32[COLS_FORMS] = {
     {2, 1, 8, 3, 0.80f, 1.50f}, {2, 1, 16, 1, 1.12f, 1.12f}, {2, 2, 8, 2, 1.33f, 2.1f},
@@ -306,47 +299,6 @@ static const ColsForm FORMS_16[COLS_FORMS] = {
     {2, 1, 8, 3, 1.00f, 1.66f}, {2, 1, 16, 1, 1.40f, 1.40f}, {2, 2, 8, 2, 1.67f, 2.35f},
     {3, 1, 16, 1, 2.10f, 2.10f}, {4, 1, 16, 1, 2.90f, 2.90f}, {4, 3, 8, 1, 4.5f, 4.5f}};
 
-static dim3 cols_grid(const ColsForm& c, Dims d, int zc) {
-    const int OW = 64 - 2 * c.K, rows = c.NW * c.R, OH = rows - 2 * (c.K - 1);
-    return dim3(d.X > 64 ? (d.X - 64 + OW - 1) / OW + 1 : 1, d.Y > rows ? (d.Y - rows + OH - 1) / OH + 1 : 1,
-                (d.Z - 2 + zc - 1) / zc);
-}
-
-// Planes per chunk of one form, and the estimated microseconds of a launch: a
-// chunk of zc planes takes zc + 2 (K - 1) steps (rounded up to the loop's
-// four), so short chunks repeat more steps and long ones leave CUs idle or a
-// last round part full; a launch also moves its planes once and costs about
-// 5 us to start and to fill the pipeline.
-struct ColsPlan {
-    int form, zc;
-    float us;
-};
-static ColsPlan cols_plan(const ColsForm* forms, int form, Dims d, size_t elem) {
-    const ColsForm& c = forms[form];
-    const double cus = cu_count(), pb = (double)d.X * d.Y * elem;
-    ColsPlan best{form, 2, 1e30f};
-    for (int steps = (2 * c.K + 3) & ~3; steps <= 140; steps += 4) {
-        const int zc = steps - 2 * (c.K - 1);
-        if (zc < 2 || pb * (steps + 4) >= 2147483648.0) continue;
-        const dim3 g = cols_grid(c, d, zc);
-        const double per_cu = (double)g.x * g.y * g.z / cus;
-        double t;
-        if (per_cu <= c.occ) {
-            const double n = ceil(per_cu);
-            t = c.occ > 1 ? c.one + (n - 1) * (c.full - c.one) / (c.occ - 1) : c.one;
-        } else if (per_cu <= 4 * c.occ) {
-            t = ceil(per_cu / c.occ - 0.5) * c.full + (per_cu / c.occ - floor(per_cu / c.occ) > 0.5 ? 0 : c.one);
-        } else {
-            t = (per_cu / c.occ + 0.5) * c.full;
-        }
-        // v and f with the planes beside the chunk, the result; 4 TB/s
-        const double memory = elem * (double)d.n() * (6.0 * (zc + 2 * c.K) / zc + 3.0) / 4.0e6;
-        const float us = (float)std::max(t * steps, memory) + 5.0f;
-        if (us < best.us) best = ColsPlan{form, zc, us};
-        if (zc >= d.Z - 2) break;
-    }
-    return best;
-}
 template <class S>
 static const ColsForm* cols_forms() {
     return std::is_same<S, F32>::value ? FORMS_F32 : FORMS_16;
@@ -355,9 +307,10 @@ static const ColsForm* cols_forms() {
 template <class S>
 static ColsPlan cols_best(std::initializer_list<int> forms, Dims d) {
     const ColsForm* F = cols_forms<S>();
+    constexpr size_t e = sizeof(typename S::T);  // v and f read, the result written
     ColsPlan best{0, 0, 1e30f};
     for (int f : forms) {
-        const ColsPlan p = cols_plan(F, f, d, sizeof(typename S::T));
+        const ColsPlan p = cols_plan(F[f], f, d, d.Z - 2, (double)d.X * d.Y * e, 6.0 * e, 3.0 * e);
         if (best.zc == 0 || p.us * F[best.form].K < best.us * F[p.form].K) best = p;
     }
     return best;
@@ -365,7 +318,7 @@ static ColsPlan cols_best(std::initializer_list<int> forms, Dims d) {
 
 template <class S, int K, int R, int NW, int WPE, bool MIDS>
 static void launch_cols_form(bool finish, const ColsArgs<S>& a, const ColsForm& c, hipStream_t stream) {
-    const dim3 grid = cols_grid(c, a.d, a.zc), block(64 * NW);
+    const dim3 grid = cols_grid(c, a.d, a.d.Z - 2, a.zc), block(64 * NW);
     if (finish) hipLaunchKernelGGL((k_gvf_cols<S, K, R, NW, WPE, true, false>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((k_gvf_cols<S, K, R, NW, WPE, false, MIDS>), grid, block, 0, stream, a);
 }

@@ -42,6 +42,8 @@
 // are not rounded (F32) or are rounded alike (SNORM16).
 #pragma once
 
+#include <math.h>
+
 #include "tsf_common.hpp"
 
 namespace tsf {
@@ -533,6 +535,57 @@ __global__ void __launch_bounds__(64 * NW, WPE) k_gvf_cols(ColsArgs<S> a) {
     __shared__ typename M::Lds lds[2];
     M m(a, lds);
     m.run();
+}
+
+// ---------------------------------------------------------------- host: form and chunk of a launch
+// A built form of a marching kernel: K steps, R rows per wave, NW waves.
+// occ: workgroups a CU holds; one, full: microseconds per step of one
+// workgroup alone on a CU and of occ of them sharing it (measured at 4 to 136
+// steps per launch, 64^3 to 512^3).
+struct ColsForm {
+    int K, R, NW, occ;
+    float one, full;
+};
+inline dim3 cols_grid(const ColsForm& c, Dims d, int planes, int zc) {
+    const int OW = 64 - 2 * c.K, rows = c.NW * c.R, OH = rows - 2 * (c.K - 1);
+    return dim3(d.X > 64 ? (d.X - 64 + OW - 1) / OW + 1 : 1, d.Y > rows ? (d.Y - rows + OH - 1) / OH + 1 : 1,
+                (planes + zc - 1) / zc);
+}
+
+// Planes per chunk of a form, and the estimated microseconds of a launch: a
+// chunk of zc planes takes zc + 2 (K - 1) steps (rounded up to the loop's
+// four), so short chunks repeat more steps and long ones leave CUs idle or a
+// last round part full; a launch also moves `once` bytes a voxel and `halo`
+// bytes that the planes beside a chunk repeat, and costs about 5 us to start
+// and to fill the pipeline.  range: bytes per plane that a chunk's buffer
+// resources cover (0: no limit from them).
+struct ColsPlan {
+    int form, zc;
+    float us;
+};
+inline ColsPlan cols_plan(const ColsForm& c, int form, Dims d, int planes, double range, double halo, double once) {
+    const double cus = cu_count();
+    ColsPlan best{form, 2, 1e30f};
+    for (int steps = (2 * c.K + 3) & ~3; steps <= 140; steps += 4) {
+        const int zc = steps - 2 * (c.K - 1);
+        if (zc < 2 || range * (steps + 4) >= 2147483648.0) continue;
+        const dim3 g = cols_grid(c, d, planes, zc);
+        const double per_cu = (double)g.x * g.y * g.z / cus;
+        double t;
+        if (per_cu <= c.occ) {
+            const double n = ceil(per_cu);
+            t = c.occ > 1 ? c.one + (n - 1) * (c.full - c.one) / (c.occ - 1) : c.one;
+        } else if (per_cu <= 4 * c.occ) {
+            t = ceil(per_cu / c.occ - 0.5) * c.full + (per_cu / c.occ - floor(per_cu / c.occ) > 0.5 ? 0 : c.one);
+        } else {
+            t = (per_cu / c.occ + 0.5) * c.full;
+        }
+        const double memory = (double)d.n() * (halo * (zc + 2 * c.K) / zc + once) / 4.0e6;  // 4 TB/s
+        const float us = (float)fmax(t * steps, memory) + 5.0f;
+        if (us < best.us) best = ColsPlan{form, zc, us};
+        if (zc >= planes) break;
+    }
+    return best;
 }
 
 }  // namespace tsf
