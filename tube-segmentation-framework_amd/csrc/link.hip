@@ -82,59 +82,93 @@ __device__ __forceinline__ float segment_mean_tdf(const float* __restrict__ T, c
 
 // linkLengths + compact: neighbours b of a with 0 < |xb - xa| < maxDistance,
 // in ascending b (the reference's order is that of its atomic increments).
-__global__ void k_link_cand(const int32_t* __restrict__ v, int count, float maxd, int32_t* __restrict__ cand,
-                            int32_t* __restrict__ ncand) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+// A wave per vertex: 64 vertices at a time, the lanes' verdicts packed by
+// ballot.
+__global__ void __launch_bounds__(256) k_link_cand(const int32_t* __restrict__ v, int count, float maxd,
+                                                   int32_t* __restrict__ cand, int32_t* __restrict__ ncand) {
+    const int lane = threadIdx.x & 63, a = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (a >= count) return;
     const F3 xa = vert(v, a);
     int32_t* row = cand + (i64)a * count;
     int n = 0;
-    for (int b = 0; b < count; b++) {
-        const float l = dist3(xa, vert(v, b));
-        if (l < maxd && l > 0.0f) row[n++] = b;
+    for (int b0 = 0; b0 < count; b0 += 64) {
+        const int b = b0 + lane;
+        bool near = false;
+        if (b < count) {
+            const float l = dist3(xa, vert(v, b));
+            near = l < maxd && l > 0.0f;
+        }
+        const unsigned long long m = __ballot(near);
+        if (near) row[n + __popcll(m & ((1ull << lane) - 1))] = b;
+        n += __popcll(m);
     }
-    ncand[a] = n;
+    if (lane == 0) ncand[a] = n;
 }
 
 // linkCenterpoints (kernels_no_3d_write.cl:753-882): among the pairs (b, c)
 // of candidates, c listed before b, the one of smallest round|ab| +
-// round|ac| (the first found on ties) whose angle at a exceeds 2 rad and
-// whose segments ab and ac both have a mean TDF >= minAvgTDF.
-__global__ void k_link_pairs(const int32_t* __restrict__ v, int count, const int32_t* __restrict__ cand,
-                             const int32_t* __restrict__ ncand, const float* __restrict__ T, Dims d, float maxd,
-                             float min_avg, int32_t* __restrict__ pair) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+// round|ac| below 2 maxDistance (the first found on ties) whose angle at a
+// exceeds 2 rad and whose segments ab and ac both have a mean TDF >=
+// minAvgTDF.  A wave per vertex: the segment test depends on one candidate
+// alone, so it is done once for each (64 at a time) and the row is packed to
+// those that pass, in order; then the lanes take the pairs of that row and the
+// least (sum, i, j) wins, which is the pair the reference's loop ends with
+// (its skips by the length found so far drop only pairs that cannot win).
+// 667 vertices: 109 + 254 us with a thread per vertex for the two kernels,
+// 7 + 25 us so.
+__global__ void __launch_bounds__(256) k_link_pairs(const int32_t* __restrict__ v, int count,
+                                                    int32_t* __restrict__ cand, const int32_t* __restrict__ ncand,
+                                                    const float* __restrict__ T, Dims d, float maxd, float min_avg,
+                                                    int32_t* __restrict__ pair) {
+    const int lane = threadIdx.x & 63, a = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (a >= count) return;
     const F3 xa = vert(v, a);
-    const int32_t* row = cand + (i64)a * count;
-    const int n = ncand[a];
-    float shortest = maxd * 2.0f;
-    int bx = -1, by = -1;
-    for (int i = 0; i < n; i++) {
-        const int b = row[i];
-        const F3 xb = vert(v, b);
+    int32_t* row = cand + (i64)a * count;
+    const int all = ncand[a];
+    int n = 0;
+    for (int i0 = 0; i0 < all; i0 += 64) {
+        const int i = i0 + lane;
+        int b = -1;
+        bool ok = false;
+        if (i < all) {
+            b = row[i];
+            const F3 xb = vert(v, b);
+            const F3 ab{xb.x - xa.x, xb.y - xa.y, xb.z - xa.z};
+            ok = !(segment_mean_tdf(T, d, xa, ab, (int)roundf(dist3(xa, xb))) < min_avg);
+        }
+        const unsigned long long m = __ballot(ok);  // after the wave's reads of row[i0 ..]
+        if (ok) row[n + __popcll(m & ((1ull << lane) - 1))] = b;
+        n += __popcll(m);
+    }
+    __threadfence_block();  // the lanes read what others packed
+    unsigned long long best = ~0ull;
+    for (int i = 1; i < n; i++) {
+        const F3 xb = vert(v, row[i]);
         const int db = (int)roundf(dist3(xa, xb));
-        if ((float)db >= shortest) continue;
-        for (int j = 0; j < i; j++) {
-            const int c = row[j];
-            if (c == b) continue;
-            const F3 xc = vert(v, c);
-            const int dc = (int)roundf(dist3(xa, xc));
-            if (!((float)(db + dc) < shortest)) continue;
-            const F3 ab{xb.x - xa.x, xb.y - xa.y, xb.z - xa.z}, ac{xc.x - xa.x, xc.y - xa.y, xc.z - xa.z};
-            const float lb = sqrtf(ab.x * ab.x + ab.y * ab.y + ab.z * ab.z);
+        const F3 ab{xb.x - xa.x, xb.y - xa.y, xb.z - xa.z};
+        const float lb = sqrtf(ab.x * ab.x + ab.y * ab.y + ab.z * ab.z);
+        for (int j = lane; j < i; j += 64) {
+            const F3 xc = vert(v, row[j]);
+            const int sum = db + (int)roundf(dist3(xa, xc));
+            const unsigned long long key =
+                ((unsigned long long)(unsigned)sum << 32) | ((unsigned)i << 16) | (unsigned)j;
+            if (!((float)sum < maxd * 2.0f) || key >= best) continue;
+            const F3 ac{xc.x - xa.x, xc.y - xa.y, xc.z - xa.z};
             const float lc = sqrtf(ac.x * ac.x + ac.y * ac.y + ac.z * ac.z);
             const float dot = (ab.x / lb) * (ac.x / lc) + (ab.y / lb) * (ac.y / lc) + (ab.z / lb) * (ac.z / lc);
-            if (acosf(dot) < 2.0f) continue;
-            if (segment_mean_tdf(T, d, xa, ab, db) < min_avg) continue;
-            if (segment_mean_tdf(T, d, xa, ac, dc) < min_avg) continue;
-            bx = b;
-            by = c;
-            shortest = (float)(db + dc);
+            if (!(acosf(dot) < 2.0f)) best = key;
         }
     }
-    pair[2 * a] = bx;
-    pair[2 * a + 1] = by;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long k = __shfl_xor(best, o);
+        best = k < best ? k : best;
+    }
+    if (lane == 0) {
+        const bool found = best != ~0ull;
+        pair[2 * a] = found ? row[(unsigned)best >> 16] : -1;
+        pair[2 * a + 1] = found ? row[(unsigned)best & 0xffffu] : -1;
+    }
 }
 
 // 2D pyramid traversal key of cell (x, y) < 2^16: sum_b (2 x_b + y_b) 4^b.
@@ -175,11 +209,11 @@ __global__ void __launch_bounds__(1024) k_link_count(const uint64_t* __restrict_
 }
 
 // The list position of every edge: the number of smaller keys (keys are
-// distinct), through LDS tiles of 1024 keys.
+// distinct), through LDS tiles of 1024 keys, four threads per edge.
 __global__ void __launch_bounds__(256) k_link_rank(const uint64_t* __restrict__ keys, const int32_t* __restrict__ pair,
                                                    int n, int32_t* __restrict__ edges, int capacity) {
     __shared__ uint64_t tile[1024];
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int s = blockIdx.x * 64 + (threadIdx.x >> 2);
     const uint64_t k = s < n ? keys[s] : NO_EDGE;
     int rank = 0;
     for (int t0 = 0; t0 < n; t0 += 1024) {
@@ -187,9 +221,12 @@ __global__ void __launch_bounds__(256) k_link_rank(const uint64_t* __restrict__ 
         for (int i = threadIdx.x; i < 1024; i += 256) tile[i] = t0 + i < n ? keys[t0 + i] : NO_EDGE;
         __syncthreads();
         const int m = min(1024, n - t0);
-        for (int i = 0; i < m; i++) rank += tile[i] < k;
+#pragma unroll 8
+        for (int i = threadIdx.x & 3; i < m; i += 4) rank += tile[i] < k;
     }
-    if (k != NO_EDGE && rank < capacity) {
+    rank += __shfl_xor(rank, 1);
+    rank += __shfl_xor(rank, 2);
+    if ((threadIdx.x & 3) == 0 && k != NO_EDGE && rank < capacity) {
         edges[2 * rank] = s >> 1;
         edges[2 * rank + 1] = pair[s];
     }
@@ -200,11 +237,17 @@ __global__ void __launch_bounds__(256) k_link_rank(const uint64_t* __restrict__ 
 // (at most `count` passes: the smallest index of a component spreads one
 // edge per pass at least) with every vertex labelled by its component's
 // smallest index; *status = 0, or 1 if the pass bound was reached first
-// (not expected).
+// (not expected).  IN_LDS: the labels live in LDS during the passes, which
+// are chains of dependent label reads (up to COMP_LDS vertices, the most the
+// centerline extraction takes: 64 KB).  667 vertices: 54 -> 29 us.
+constexpr int COMP_LDS = 16384;
+template <bool IN_LDS>
 __global__ void __launch_bounds__(1024) k_components(const int32_t* __restrict__ edges, int n_edges, int count,
-                                                     int32_t* __restrict__ L, int32_t* __restrict__ S,
+                                                     int32_t* __restrict__ labels, int32_t* __restrict__ S,
                                                      int32_t* __restrict__ status) {
     __shared__ int changed;
+    __shared__ int32_t shared_labels[IN_LDS ? COMP_LDS : 1];
+    int32_t* L = IN_LDS ? shared_labels : labels;
     for (int i = threadIdx.x; i < count; i += 1024) {
         L[i] = i;
         S[i] = 0;
@@ -239,7 +282,10 @@ __global__ void __launch_bounds__(1024) k_components(const int32_t* __restrict__
         __syncthreads();
         if (!c || pass >= count) break;
     }
-    for (int i = threadIdx.x; i < count; i += 1024) atomicAdd(&S[L[i]], 1);
+    for (int i = threadIdx.x; i < count; i += 1024) {
+        if (IN_LDS) labels[i] = L[i];
+        atomicAdd(&S[L[i]], 1);
+    }
     if (threadIdx.x == 0) *status = changed ? 1 : 0;
 }
 
@@ -306,13 +352,13 @@ tsf_status tsf_link_centerpoints(const int32_t* vertices, int32_t count, const f
     uint64_t* keys = (uint64_t*)p;
     p += (2 * c * sizeof(uint64_t) + 255) & ~(size_t)255;
     int32_t* dcount = (int32_t*)p;
-    hipLaunchKernelGGL(k_link_cand, blocks(count, 64), 64, 0, stream, vertices, count, max_distance, cand, ncand);
-    hipLaunchKernelGGL(k_link_pairs, blocks(count, 64), 64, 0, stream, vertices, count, cand, ncand, tdf, d,
+    hipLaunchKernelGGL(k_link_cand, blocks(count, 4), 256, 0, stream, vertices, count, max_distance, cand, ncand);
+    hipLaunchKernelGGL(k_link_pairs, blocks(count, 4), 256, 0, stream, vertices, count, cand, ncand, tdf, d,
                        max_distance, min_mean_tdf, pair);
     hipLaunchKernelGGL(k_link_keys, blocks(2 * (i64)count, 256), 256, 0, stream, pair, count, keys);
     hipLaunchKernelGGL(k_link_count, 1, 1024, 0, stream, keys, 2 * count, dcount);
     if (capacity > 0)
-        hipLaunchKernelGGL(k_link_rank, blocks(2 * (i64)count, 256), 256, 0, stream, keys, pair, 2 * count, edges,
+        hipLaunchKernelGGL(k_link_rank, blocks(2 * (i64)count, 64), 256, 0, stream, keys, pair, 2 * count, edges,
                            capacity);
     TSF_TRY(check_launch(W));
     int32_t total = 0;
@@ -333,7 +379,10 @@ tsf_status tsf_graph_components(const int32_t* edges, int32_t n_edges, int32_t c
     Scratch sc;
     TSF_TRY(sc.get(nullptr, 0, 256, W));
     int32_t* status = (int32_t*)sc.ptr;
-    hipLaunchKernelGGL(k_components, 1, 1024, 0, stream, edges, n_edges, count, labels, sizes, status);
+    if (count <= COMP_LDS)
+        hipLaunchKernelGGL(k_components<true>, 1, 1024, 0, stream, edges, n_edges, count, labels, sizes, status);
+    else
+        hipLaunchKernelGGL(k_components<false>, 1, 1024, 0, stream, edges, n_edges, count, labels, sizes, status);
     TSF_TRY(check_launch(W));
     int32_t h = 0;
     hipError_t e = hipMemcpyAsync(&h, status, sizeof h, hipMemcpyDeviceToHost, stream);

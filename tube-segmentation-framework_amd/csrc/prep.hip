@@ -228,6 +228,18 @@ __global__ void k_candidates(const float* __restrict__ tdf, uint8_t* __restrict_
     for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x)
         mask[i] = tdf[i] < thr ? 0 : 1;
 }
+// The same for four voxels a thread and access (tdf 16-byte, mask 4-byte
+// aligned; the remainder by the first threads).  105 M voxels: 151 -> 100 us.
+__global__ void k_candidates4(const float* __restrict__ tdf, uint8_t* __restrict__ mask, i64 n, float thr) {
+    const i64 n4 = n / 4, step = (i64)gridDim.x * blockDim.x, t = blockIdx.x * (i64)blockDim.x + threadIdx.x;
+    for (i64 i = t; i < n4; i += step) {
+        const float4 v = reinterpret_cast<const float4*>(tdf)[i];
+        const unsigned m = (v.x < thr ? 0u : 1u) | (v.y < thr ? 0u : 1u << 8) | (v.z < thr ? 0u : 1u << 16) |
+                           (v.w < thr ? 0u : 1u << 24);
+        reinterpret_cast<unsigned*>(mask)[i] = m;
+    }
+    if (t < n - 4 * n4) mask[4 * n4 + t] = tdf[4 * n4 + t] < thr ? 0 : 1;
+}
 
 static unsigned grid1d(i64 n, int block) {
     i64 g = (n + block - 1) / block;
@@ -375,7 +387,10 @@ tsf_status tsf_candidates(const float* tdf, uint8_t* mask, int64_t count, float 
     if (!tdf || !mask) return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: NULL buffer", W);
     if (count < 0) return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: negative count", W);
     if (count == 0) return TSF_OK;
-    hipLaunchKernelGGL(k_candidates, grid1d(count, 256), 256, 0, stream, tdf, mask, (i64)count, threshold);
+    if ((uintptr_t)tdf % 16 == 0 && (uintptr_t)mask % 4 == 0)
+        hipLaunchKernelGGL(k_candidates4, grid1d((count + 3) / 4, 256), 256, 0, stream, tdf, mask, (i64)count, threshold);
+    else
+        hipLaunchKernelGGL(k_candidates, grid1d(count, 256), 256, 0, stream, tdf, mask, (i64)count, threshold);
     return check_launch(W);
 }
 

@@ -63,72 +63,172 @@ __global__ void k_do_eigen_points(const float* __restrict__ Fx, const float* __r
     }
 }
 
-// findCandidateCenterpoints2, kernels_no_3d_write.cl:1019-1084.
+// findCandidateCenterpoints2, kernels_no_3d_write.cl:1019-1084: a candidate
+// is rejected if a voxel at offset r, 0 < |r| < maxD, whose direction lies
+// within 0.5 rad of the plane normal to e1, has a smaller magnitude.
+//
+// The angle test of the reference, theta = acos(r/|r| . p/|p|) with p = r -
+// e1 (e1 . r), is sin^2 of the angle between r and that plane: for a unit e1
+// theta < 0.5 exactly when (e1 . r)^2 < sin^2(0.5) |r|^2.  Offsets clear of
+// that bound by 1e-4 |r|^2 (the float expressions are within 1e-5 of it) are
+// decided by it; the others, and all of them when e1 is not of unit length to
+// 1e-5, by the reference's own expressions.
+struct NmsCandidate {
+    int x, y, z, maxD;
+    float ex, ey, ez, wp;
+    bool unit;
+};
+__device__ __forceinline__ bool nms_in_plane(const NmsCandidate& q, int a, int b, int c) {
+    const float rx = (float)a, ry = (float)b, rz = (float)c;
+    const float dp = q.ex * rx + q.ey * ry + q.ez * rz;
+    const float r2 = (float)(a * a + b * b + c * c), d2 = dp * dp;
+    if (q.unit && d2 < 0.2297488f * r2) return true;
+    if (q.unit && d2 > 0.2299488f * r2) return false;
+    const float px = rx - q.ex * dp, py = ry - q.ey * dp, pz = rz - q.ez * dp;
+    const float lr = sqrtf(rx * rx + ry * ry + rz * rz);
+    const float lp = sqrtf(px * px + py * py + pz * pz);
+    const float cs = (rx / lr) * (px / lp) + (ry / lr) * (py / lp) + (rz / lr) * (pz / lp);
+    return acosf(cs) < 0.5f;
+}
+template <class S>
+__device__ __forceinline__ bool nms_beaten(const NmsCandidate& q, const Field<S>& F, const Dims& d, int a, int b,
+                                           int c) {
+    const int r2 = a * a + b * b + c * c;
+    if (r2 == 0 || r2 >= q.maxD * q.maxD || !nms_in_plane(q, a, b, c)) return false;
+    const int nx = clampi(q.x + a, 0, d.X - 1), ny = clampi(q.y + b, 0, d.Y - 1), nz = clampi(q.z + c, 0, d.Z - 1);
+    return F.mag(d.at(nx, ny, nz)) < q.wp;
+}
+// A thread solves for its candidate's e1 and looks at the 26 voxels next to
+// it, which rejects most candidates off the axis; the survivors with a wider
+// reach are collected in LDS and a wave searches each of them, 64 offsets at
+// a time.  192298 candidates of tubes up to radius 8 (reach up to 8: 4913
+// offsets): 3267 us with a thread per candidate and the reference's
+// expressions at every offset, 93 us so.
 template <class S>
 __global__ void __launch_bounds__(256) k_candidate_nms(const float* __restrict__ radius, Field<S> F, Dims d,
                                                        const int32_t* __restrict__ pos, i64 count, int cap,
                                                        uint8_t* __restrict__ out) {
-    i64 t = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    const int x = pos[3 * t], y = pos[3 * t + 1], z = pos[3 * t + 2];
-    if (x < 0 || y < 0 || z < 0 || x >= d.X || y >= d.Y || z >= d.Z) return;  // not a voxel: ignored
-    const float rr = radius[d.at(x, y, z)];
-    const int maxD = (int)fmaxf(fminf(roundf(rr), (float)cap), 1.0f);
-    float H[3][3], V[3][3], ev[3];
-    hessian<true>(F, d, x, y, z, H);
-    eigen3(H, V, ev);
-    const float e1x = V[0][0], e1y = V[1][0], e1z = V[2][0];
-    const float wp = F.mag(d.at(x, y, z));
-    bool invalid = false;
-    for (int a = -maxD; a <= maxD; a++)
-        for (int b = -maxD; b <= maxD; b++)
-            for (int c = -maxD; c <= maxD; c++) {
-                if (a == 0 && b == 0 && c == 0) continue;
-                const float rx = (float)a, ry = (float)b, rz = (float)c;
-                const float dp = e1x * rx + e1y * ry + e1z * rz;
-                const float px = rx - e1x * dp, py = ry - e1y * dp, pz = rz - e1z * dp;
-                const float lr = sqrtf(rx * rx + ry * ry + rz * rz);
-                const float lp = sqrtf(px * px + py * py + pz * pz);
-                const float cs = (rx / lr) * (px / lp) + (ry / lr) * (py / lp) + (rz / lr) * (pz / lp);
-                const float theta = acosf(cs);
-                if (theta < 0.5f && lr < (float)maxD) {
-                    const int nx = clampi(x + a, 0, d.X - 1), ny = clampi(y + b, 0, d.Y - 1),
-                              nz = clampi(z + c, 0, d.Z - 1);
-                    if (F.mag(d.at(nx, ny, nz)) < wp) invalid = true;
-                }
+    __shared__ NmsCandidate list[256];
+    __shared__ int n;
+    if (threadIdx.x == 0) n = 0;
+    __syncthreads();
+    const i64 t = blockIdx.x * (i64)blockDim.x + threadIdx.x;
+    if (t < count) {
+        NmsCandidate q;
+        q.x = pos[3 * t];
+        q.y = pos[3 * t + 1];
+        q.z = pos[3 * t + 2];
+        // a position that is not a voxel is ignored
+        if (q.x >= 0 && q.y >= 0 && q.z >= 0 && q.x < d.X && q.y < d.Y && q.z < d.Z) {
+            const i64 i = d.at(q.x, q.y, q.z);
+            q.maxD = (int)fmaxf(fminf(roundf(radius[i]), (float)cap), 1.0f);
+            bool valid = true;
+            if (q.maxD > 1) {
+                float H[3][3], V[3][3], ev[3];
+                hessian<true>(F, d, q.x, q.y, q.z, H);
+                eigen3(H, V, ev);
+                q.ex = V[0][0];
+                q.ey = V[1][0];
+                q.ez = V[2][0];
+                q.wp = F.mag(i);
+                q.unit = fabsf(q.ex * q.ex + q.ey * q.ey + q.ez * q.ez - 1.0f) < 1e-5f;
+                for (int c = -1; c <= 1; c++)
+                    for (int b = -1; b <= 1; b++)
+                        for (int a = -1; a <= 1; a++)
+                            if (nms_beaten(q, F, d, a, b, c)) valid = false;
             }
-    out[d.at(x, y, z)] = invalid ? 0 : 1;
+            if (valid && q.maxD > 2) list[atomicAdd(&n, 1)] = q;
+            else out[i] = valid;
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    for (int k = threadIdx.x >> 6; k < n; k += 4) {
+        const NmsCandidate q = list[k];
+        const int m = q.maxD - 1, w = 2 * m + 1, total = w * w * w;  // |r| < maxD: components to maxD - 1
+        bool beaten = false;
+        for (int j = lane; j - lane < total && !beaten; j += 64) {
+            const int c = j / (w * w), r = j - c * (w * w), b = r / w, a = r - b * w;
+            beaten = __any(j < total && nms_beaten(q, F, d, a - m, b - m, c - m));
+        }
+        if (lane == 0) out[d.at(q.x, q.y, q.z)] = !beaten;
+    }
 }
 
-// dd, kernels_no_3d_write.cl:970-1004 (in-range voxels only).
-__global__ void k_cube_max(const float* __restrict__ tdf, const uint8_t* __restrict__ cand, Dims d, int cube, int cx,
-                           int cy, int cz, uint8_t* __restrict__ out) {
-    i64 cell = blockIdx.x * (i64)blockDim.x + threadIdx.x;
-    if (cell >= (i64)cx * cy * cz) return;
-    const int gx = (int)(cell % cx), gy = (int)((cell / cx) % cy), gz = (int)(cell / ((i64)cx * cy));
-    float best = 0.0f;
-    i64 bi = -1;
-    for (int a = 0; a < cube; a++) {
-        const int x = gx * cube + a;
-        if (x >= d.X) break;
-        for (int b = 0; b < cube; b++) {
-            const int y = gy * cube + b;
-            if (y >= d.Y) break;
-            for (int c = 0; c < cube; c++) {
-                const int z = gz * cube + c;
-                if (z >= d.Z) break;
-                const i64 i = d.at(x, y, z);
-                if (cand[i] == 1) {
-                    const float t = tdf[i];
-                    if (t > best) {
-                        best = t;
-                        bi = i;
-                    }
+// dd, kernels_no_3d_write.cl:970-1004 (in-range voxels only): of every cell's
+// candidates the one with the greatest TDF above 0, of equal ones the first in
+// x, y, z order (z innermost).  A workgroup takes whole cells of one (y, z)
+// row of cells: a thread finds the best of each of its V columns (rows of the
+// mask are read as they lie, V bytes a thread and access, eight accesses in
+// flight), then the first column of a cell takes the best of its columns in x
+// order.  V = 4 where rows are whole words.  Candidates are few, so the mask's
+// bytes bound it: 400 x 512 x 512, cube 5: 124 us with a thread per cell, 170
+// with V = 1, 59 with V = 4.
+constexpr int CM_T = 128;
+template <int V>
+__global__ void __launch_bounds__(CM_T) k_cube_max(const float* __restrict__ tdf, const uint8_t* __restrict__ cand,
+                                                   Dims d, int cube, int cols, uint8_t* __restrict__ out) {
+    __shared__ float top[CM_T * V];
+    __shared__ int at[CM_T * V];  // z * cube + y within the cell
+    const int xl = threadIdx.x * V, x0 = blockIdx.x * cols, x = x0 + xl;
+    const int y0 = blockIdx.y * cube, z0 = blockIdx.z * cube;
+    float best[V];
+    int bi[V];
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+        best[e] = 0.0f;
+        bi[e] = -1;
+    }
+    if (xl < cols && x < d.X) {
+        const int ny = min(cube, d.Y - y0), nz = min(cube, d.Z - z0), n = ny * nz;
+        int b = 0, c = 0;
+        for (int j = 0; j < n; j += 8) {
+            i64 i[8];
+            unsigned m[8];
+            int q[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                q[k] = c * cube + b;
+                i[k] = d.at(x, y0 + b, z0 + c);
+                m[k] = V == 4 ? *reinterpret_cast<const unsigned*>(cand + i[k]) : cand[i[k]];
+                if (j + k >= n) m[k] = 0;  // a repeat of the last voxel
+                c++;
+                if (c == nz) {
+                    c = b + 1 < ny ? 0 : nz - 1;
+                    b = b + 1 < ny ? b + 1 : b;
                 }
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                if (m[k] == 0) continue;
+#pragma unroll
+                for (int e = 0; e < V; e++)
+                    if (((m[k] >> (8 * e)) & 0xffu) == 1u) {
+                        const float t = tdf[i[k] + e];
+                        if (t > best[e]) {
+                            best[e] = t;
+                            bi[e] = q[k];
+                        }
+                    }
             }
         }
     }
-    if (bi >= 0) out[bi] = 1;
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+        top[xl + e] = best[e];
+        at[xl + e] = bi[e];
+    }
+    __syncthreads();
+    for (int l = threadIdx.x * cube; l < cols && x0 + l < d.X; l += CM_T * cube) {
+        float m = 0.0f;
+        int k = -1;
+        for (int a = l; a < l + cube; a++)
+            if (top[a] > m) {
+                m = top[a];
+                k = a;
+            }
+        if (k >= 0) out[d.at(x0 + k, y0 + at[k] % cube, z0 + at[k] / cube)] = 1;
+    }
 }
 
 }  // namespace tsf
@@ -239,10 +339,13 @@ tsf_status tsf_cube_max(const float* tdf, const uint8_t* candidates, tsf_dims di
     TSF_TRY(check_dims(dims, 1, W));
     if (cube < 1 || cube > 64) return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: cube size out of [1, 64]", W);
     Dims d = D(dims);
-    const int cx = (d.X + cube - 1) / cube, cy = (d.Y + cube - 1) / cube, cz = (d.Z + cube - 1) / cube;
-    const i64 cells = (i64)cx * cy * cz;
-    hipLaunchKernelGGL(k_cube_max, (unsigned)((cells + 255) / 256), 256, 0, stream, tdf, candidates, d, cube, cx, cy, cz,
-                       out);
+    const bool words = d.X % 4 == 0 && (uintptr_t)candidates % 4 == 0;
+    const int unit = words ? 4 * cube : cube, cols = (words ? 4 : 1) * CM_T / unit * unit;  // whole cells and words
+    const dim3 grid((d.X + cols - 1) / cols, (d.Y + cube - 1) / cube, (d.Z + cube - 1) / cube);
+    if (words)
+        hipLaunchKernelGGL(k_cube_max<4>, grid, CM_T, 0, stream, tdf, candidates, d, cube, cols, out);
+    else
+        hipLaunchKernelGGL(k_cube_max<1>, grid, CM_T, 0, stream, tdf, candidates, d, cube, cols, out);
     return check_launch(W);
 }
 
