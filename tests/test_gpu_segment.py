@@ -77,3 +77,40 @@ def test_segment_reads_16bit_fields(tsf, orc):
     got, passes = run_device(tsf, cl, r, Fq, storage=(tsf.STORAGE_SN16, 1.0))
     exp, opasses = orc.segment_inverse_gradient(cl, r, Fq)
     assert passes == opasses and np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("nx,half,step", [(8, 16, 1), (13, 16, 1), (4, 4, 1), (5, 1, 1), (68, 8, 2)],
+                         ids=["two-batches", "odd-rows", "dense", "dense-odd", "sparse-seeds"])
+def test_segment_lists_and_dense_passes(tsf, orc, nx, half, step):
+    """Growing on lists over more than one batch of passes, and volumes whose
+    candidates overflow the lists (seeds of half size 1..4 in a volume little
+    larger than them), at row lengths with and without whole words."""
+    side = 2 * half + 2
+    shape = (side, side + 1, nx)
+    F = tube_field(shape, 0.75 * half)
+    cl = np.zeros(shape, np.uint8)
+    cl[side // 2, side // 2, ::step] = 1
+    r = np.full(shape, 2.0 if half > 4 else 2.0 * half, np.float32)
+    got, passes = run_device(tsf, cl, r, F)
+    exp, opasses = orc.segment_inverse_gradient(cl, r, F)
+    print(f"{shape}: {int(got.sum())} voxels, {passes} passes (oracle {opasses})")
+    assert passes == opasses and np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("seed", [5, 6])
+def test_segment_direction_ties_vs_oracle(tsf, orc, seed):
+    """Fields of small whole numbers: equal and zero components, zero vectors
+    and vectors far from unit length, where the direction that a neighbour
+    points at hangs on rounding and on the order of the 26."""
+    g = np.random.default_rng(seed)
+    shape = (24, 26, 28)
+    F = np.zeros((4,) + shape, np.float32)
+    F[:3] = g.integers(-2, 3, (3,) + shape)
+    F[3] = g.choice([0.5, 1.0, 1.5, 3.0], shape)
+    F[:3, :, :, 14:] *= np.float32(1e-33) if seed == 5 else np.float32(1.1)
+    cl = (g.random(shape) < 0.01).astype(np.uint8)
+    r = g.uniform(1.0, 5.0, shape).astype(np.float32)
+    got, passes = run_device(tsf, cl, r, F)
+    exp, opasses = orc.segment_inverse_gradient(cl, r, F)
+    print(f"{int(cl.sum())} centerline voxels -> {int(got.sum())}, {passes} passes (oracle {opasses})")
+    assert passes == opasses and np.array_equal(got, exp)
