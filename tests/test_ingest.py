@@ -98,6 +98,21 @@ def test_crop_scan_lines_vs_oracle(tsf, orc, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(33, 5, 260), (32, 4, 256), (65, 7, 64), (31, 9, 4), (40, 6, 257)], ids=str)
+def test_threshold_scan_sparse_hits_vs_oracle(tsf, orc, shape):
+    """A few voxels above the threshold at the ends of rows, waves and chunks
+    of planes, with four voxels per lane and with one."""
+    Z, Y, X = shape
+    for dt in TYPES:
+        v = np.zeros(shape, dt)
+        for z, y, x in [(0, 0, 0), (Z - 1, Y - 1, X - 1), (min(31, Z - 1), 1, X - 2), (Z // 2, Y - 1, X // 2)]:
+            v[z, y, x] = 100
+        d = tsf.DeviceArray.from_host(v)
+        for got, exp in zip(tsf.crop_scan_lines(d, tsf.CROP_THRESHOLD, 99.0), orc.crop_scan_lines(v, 0, 99.0)):
+            assert (got == exp).all(), np.dtype(dt).name
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt", TYPES, ids=lambda d: np.dtype(d).name)
 def test_to_float_region_vs_oracle(tsf, orc, dt):
     rng = np.random.default_rng(9)
