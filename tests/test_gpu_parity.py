@@ -274,6 +274,40 @@ def test_gvf_fmg(tsf, orc, shape, levels):
     assert np.all(norms[:, 1:] <= norms[:, :-1] * 1.0001)
 
 
+@pytest.mark.parametrize("shape,levels,sweeps", [
+    ((4, 5, 6), 0, (1, 2, 2)), ((9, 10, 11), 2, (1, 2, 2)), ((12, 17, 21), 1, (2, 0, 1)), ((8, 40, 33), 2, (0, 1, 1)),
+    ((16, 16, 66), 2, (1, 1, 0)), ((30, 5, 24), 2, (1, 0, 0)), ((13, 12, 7), 1, (3, 1, 1))], ids=str)
+def test_gvf_fmg_shapes_and_sweeps(tsf, orc, shape, levels, sweeps):
+    """Rows whose last cell starts a quad, ends one or lies inside it, extents
+    of 4 and 5 (each boundary mirrors the other's neighbour), and sweep counts
+    of zero, after which every cell of a grid is read and not just the black
+    ones.  The arithmetic and its order are the oracle's: equal bits."""
+    F = _field_from(orc, phantom(shape, 9), fmax=0.2)
+    f, out = tsf.Field.from_host(F), tsf.Field(shape)
+    tsf.gvf_fmg(f, out, 0.15, 2, levels, *sweeps)
+    exp = orc.gvf_fmg(F, 0.15, 2, *sweeps, levels, "f32")
+    assert np.array_equal(out.download(), exp)
+
+
+def test_gvf_fmg_one_component_at_a_time(tsf):
+    """Above 2^27 cells the components share one set of buffers: what one
+    leaves there must not reach the next, so permuted components (with a zero
+    one, which keeps the rounding of |F|^2) give permuted results."""
+    shape = (513, 512, 512)
+    g = np.random.default_rng(12)
+    a, b = (np.resize(g.uniform(-0.2, 0.2, (9, 64, 512)).astype(np.float32), shape) for _ in range(2))
+    o = np.zeros(shape, np.float32)
+    got = []
+    for comps in ((a, b, o), (b, o, a)):
+        f, out = tsf.Field(shape), tsf.Field(shape)
+        for d, c in zip(f.planes, comps):
+            d.upload(c)
+        tsf.gvf_fmg(f, out, 0.15, 1, 1)
+        got.append([p.download() for p in out.planes[:3]])
+    assert np.array_equal(got[0][0], got[1][2]) and np.array_equal(got[0][1], got[1][0])
+    assert not got[0][2].any() and not got[1][1].any()
+
+
 # ------------------------------------------------------------------ eigen / TDF
 def _gvf_field(orc, shape, seed, iters=40, mu=0.1):
     F = _field_from(orc, phantom(shape, seed))

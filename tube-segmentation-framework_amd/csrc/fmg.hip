@@ -11,6 +11,23 @@
 // does not change between cycles.  Arithmetic is float in the reference's
 // operation order; the smoother divides with an IEEE division where the
 // reference uses native_divide.
+//
+// Layout: every grid is kept as two arrays, its red cells (x + y + z even)
+// and its black ones, rows padded to four elements.  A half-sweep then reads
+// the other colour, r and s of its own and writes its own: half the bytes of
+// whole grids, every lane at work, in place.  The mirror of a boundary cell
+// (0 -> 2, N-1 -> N-3) has the cell's colour, so the boundary cells are
+// stored by the thread that computes their mirror.  A red half-sweep does not
+// read red cells, so what precedes one (zeroing, prolongation) sets the black
+// cells only.
+//
+// The components do not depend on each other: grids up to 2^22 cells run all
+// three in one launch (a half-sweep of 64^3 cells takes 3 us for one and for
+// three), larger ones a component at a time, so that a phase's r, v and s
+// (201 MB at 256^3) can stay in the last-level cache.  Grids above 2^27 cells
+// keep one component's buffers only and run the cycles one after another.
+//
+// 256^3, two levels, 10 cycles: 27.7 ms on whole grids, 15.1 ms so.
 #include <math.h>
 #include <vector>
 
@@ -18,124 +35,377 @@
 
 namespace tsf {
 
-#define STENCIL_GRID(d) dim3(((d).X + 63) / 64, ((d).Y + 3) / 4, (d).Z), dim3(64, 4)
+// One grid: extents, elements per row and colour, cells per colour.
+struct Grid {
+    Dims d;
+    int xs;
+    i64 m;
+    explicit Grid(Dims e) : d(e), xs((((e.X + 1) / 2) + 3) & ~3), m((i64)xs * e.Y * e.Z) {}
+    __host__ __device__ i64 row(int y, int z) const { return (i64)xs * ((i64)y + (i64)d.Y * z); }
+};
+// A colour-split array is its red cells followed by its black ones.
+struct Trio {
+    float* p[3];
+};
 
-__device__ __forceinline__ bool in_dims(const Dims& d, int x, int y) { return x < d.X && y < d.Y; }
-
-__global__ void k_sqrmag(const float* __restrict__ fx, const float* __restrict__ fy, const float* __restrict__ fz,
-                         float* __restrict__ s, i64 n) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x)
-        s[i] = fx[i] * fx[i] + fy[i] * fy[i] + fz[i] * fz[i];
+__device__ __forceinline__ void ld4(float (&v)[4], const float* p) { __builtin_memcpy(v, p, 16); }
+__device__ __forceinline__ void ld4a(float (&v)[4], const float* p) {
+    const float4 q = *reinterpret_cast<const float4*>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+__device__ __forceinline__ void st4a(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+// the array that holds the even (odd) x of a row: red cells have x + y + z even
+__device__ __forceinline__ const float* even_x(const Grid& g, const float* a, int y, int z) {
+    return a + g.row(y, z) + (((y + z) & 1) ? g.m : 0);
+}
+__device__ __forceinline__ const float* odd_x(const Grid& g, const float* a, int y, int z) {
+    return a + g.row(y, z) + (((y + z) & 1) ? 0 : g.m);
+}
+// thread -> quad i (elements i .. i + 3 of a row of each colour) and row y
+__device__ __forceinline__ bool quad_of(int xs, int rows, int& i, int& y) {
+    const int q = xs >> 2, t = (int)(blockIdx.x * 256 + threadIdx.x);
+    y = t / q;
+    i = 4 * (t - y * q);
+    return y < rows;
+}
+static dim3 quad_grid(int xs, int rows, int planes, int comps) {
+    return dim3((unsigned)(((i64)(xs >> 2) * rows + 255) / 256), (unsigned)planes, (unsigned)comps);
 }
 
-// fmgResidual, kernels_no_3d_write.cl:2303-2348 (finest grid, h = 1).
-__global__ void k_fmg_residual(const float* __restrict__ Fx, const float* __restrict__ Fy,
-                               const float* __restrict__ Fz, const float* __restrict__ f, Dims d, float mu, int comp,
-                               float* __restrict__ r) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(d, x, y)) return;
-    const i64 q = d.at(remap(x, d.X), remap(y, d.Y), remap(z, d.Z));
-    const i64 sy = d.X, sz = (i64)d.X * d.Y;
-    const float fx = Fx[q], fy = Fy[q], fz = Fz[q];
-    const float v0 = comp == 0 ? fx : (comp == 1 ? fy : fz);
-    const float sq = fx * fx + fy * fy + fz * fz;
-    const float c = f[q];
-    float nb = f[q + 1];
-    nb = nb + f[q - 1];
-    nb = nb + f[q + sy];
-    nb = nb + f[q - sy];
-    nb = nb + f[q + sz];
-    nb = nb + f[q - sz];
-    const float residue = (mu * (nb - 6.0f * c)) / (1.0f * 1.0f);
-    r[d.at(x, y, z)] = -sq * v0 - (residue - sq * c);
+// s = |F|^2
+__global__ void __launch_bounds__(256) k_sqrmag(const float* __restrict__ fx, const float* __restrict__ fy,
+                                                const float* __restrict__ fz, Grid g, float* __restrict__ s) {
+    int i, y;
+    if (!quad_of(g.xs, g.d.Y, i, y)) return;
+    const int z = blockIdx.y;
+    const int odd = (y + z) & 1;
+    float e[2][4];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int x = 2 * i + j;
+        const i64 q = g.d.at(min(x, g.d.X - 1), y, z);
+        e[j & 1][j >> 1] = x < g.d.X ? fx[q] * fx[q] + fy[q] * fy[q] + fz[q] * fz[q] : 0.0f;
+    }
+    float* o = s + g.row(y, z) + i;
+    st4a(o + (odd ? g.m : 0), e[0]);
+    st4a(o + (odd ? 0 : g.m), e[1]);
 }
 
-__device__ __forceinline__ float gs_value(const float* __restrict__ v, const float* __restrict__ r,
-                                          const float* __restrict__ s, i64 q, i64 sy, i64 sz, float mu, float h) {
-    float nb = v[q + 1];
-    nb = nb + v[q - 1];
-    nb = nb + v[q + sy];
-    nb = nb + v[q - sy];
-    nb = nb + v[q + sz];
-    nb = nb + v[q - sz];
-    const float num = 2.0f * mu * nb - 2.0f * h * h * r[q];
-    const float den = 12.0f * mu + h * h * s[q];
+// fmgResidual, kernels_no_3d_write.cl:2303-2348 (finest grid, h = 1); F_c and
+// f are plain arrays, |F|^2 comes from s.  Rows past X get zeros.
+__device__ __forceinline__ float fmg_residual_of(float fc, float c, float sq, float nb, float mu) {
+    const float residue = mu * (nb - 6.0f * c);
+    return -sq * fc - (residue - sq * c);
+}
+__global__ void __launch_bounds__(256) k_fmg_residual(const float* __restrict__ Fc, const float* __restrict__ f,
+                                                      const float* __restrict__ s, Grid g, float mu,
+                                                      float* __restrict__ r) {
+    int i, y;
+    if (!quad_of(g.xs, g.d.Y, i, y)) return;
+    const int z = blockIdx.y, X = g.d.X;
+    const int py = remap(y, g.d.Y), pz = remap(z, g.d.Z);
+    const i64 sy = X, sz = (i64)X * g.d.Y, q = g.d.at(2 * i, py, pz);  // rows py, pz are interior: q - 1 .. q + 8 exist
+    auto at = [&](int x) {  // the value at column x, read apart
+        const i64 k = g.d.at(x, py, pz);
+        float nb = f[k + 1];
+        nb = nb + f[k - 1];
+        nb = nb + f[k + sy];
+        nb = nb + f[k - sy];
+        nb = nb + f[k + sz];
+        nb = nb + f[k - sz];
+        const float* sr = (x & 1) ? odd_x(g, s, py, pz) : even_x(g, s, py, pz);
+        return fmg_residual_of(Fc[k], f[k], sr[x >> 1], nb, mu);
+    };
+    float e[2][4];
+    if (2 * i + 7 < X) {
+        float c[10], yp[8], ym[8], zp[8], zm[8], fc[8], se[4], so[4];
+        __builtin_memcpy(c + 1, f + q, 32);
+        c[0] = f[q - 1];
+        c[9] = f[q + 8];
+        __builtin_memcpy(yp, f + q + sy, 32);
+        __builtin_memcpy(ym, f + q - sy, 32);
+        __builtin_memcpy(zp, f + q + sz, 32);
+        __builtin_memcpy(zm, f + q - sz, 32);
+        __builtin_memcpy(fc, Fc + q, 32);
+        ld4a(se, even_x(g, s, py, pz) + i);
+        ld4a(so, odd_x(g, s, py, pz) + i);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            float nb = c[j + 2];
+            nb = nb + c[j];
+            nb = nb + yp[j];
+            nb = nb + ym[j];
+            nb = nb + zp[j];
+            nb = nb + zm[j];
+            e[j & 1][j >> 1] = fmg_residual_of(fc[j], c[j + 1], (j & 1) ? so[j >> 1] : se[j >> 1], nb, mu);
+        }
+        if (i == 0) e[0][0] = e[0][1];
+        if (2 * i + 7 == X - 1) e[1][3] = e[1][2];
+    } else {
+        for (int j = 0; j < 8; j++) e[j & 1][j >> 1] = 2 * i + j < X ? at(remap(2 * i + j, X)) : 0.0f;
+    }
+    const int odd = (y + z) & 1;
+    float* o = r + g.row(y, z) + i;
+    st4a(o + (odd ? g.m : 0), e[0]);
+    st4a(o + (odd ? 0 : g.m), e[1]);
+}
+
+// GVFgaussSeidel / GVFgaussSeidel2 (the half-sweeps), kernels_no_3d_write.cl:
+// 2071-2150: the cells of colour BLACK from the other colour.
+__device__ __forceinline__ float gs_value(float nb, float r, float s, float mu, float h) {
+    const float num = 2.0f * mu * nb - 2.0f * h * h * r;
+    const float den = 12.0f * mu + h * h * s;
     return num / den;
 }
-
-// GVFgaussSeidel (red half-sweep), kernels_no_3d_write.cl:2071-2107.
-__global__ void k_gs_red(const float* __restrict__ v, const float* __restrict__ r, const float* __restrict__ s,
-                         Dims d, float mu, float h, float* __restrict__ t) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(d, x, y)) return;
-    const int px = remap(x, d.X), py = remap(y, d.Y), pz = remap(z, d.Z);
-    if (((px + py + pz) & 1) != 0) return;
-    t[d.at(x, y, z)] = gs_value(v, r, s, d.at(px, py, pz), d.X, (i64)d.X * d.Y, mu, h);
-}
-
-// GVFgaussSeidel2 (black half-sweep; red cells copy the remapped value),
-// kernels_no_3d_write.cl:2109-2150.
-__global__ void k_gs_black(const float* __restrict__ t, const float* __restrict__ r, const float* __restrict__ s,
-                           Dims d, float mu, float h, float* __restrict__ v) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(d, x, y)) return;
-    const int px = remap(x, d.X), py = remap(y, d.Y), pz = remap(z, d.Z);
-    const i64 q = d.at(px, py, pz);
-    v[d.at(x, y, z)] = (((px + py + pz) & 1) == 0) ? t[q] : gs_value(t, r, s, q, d.X, (i64)d.X * d.Y, mu, h);
-}
-
-// residual, kernels_no_3d_write.cl:2268-2301.
-__global__ void k_residual(const float* __restrict__ r, const float* __restrict__ v, const float* __restrict__ s,
-                           Dims d, float mu, float h, float* __restrict__ p) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(d, x, y)) return;
-    const i64 q = d.at(remap(x, d.X), remap(y, d.Y), remap(z, d.Z));
-    const i64 sy = d.X, sz = (i64)d.X * d.Y;
-    const float c = v[q];
-    float nb = v[q + 1];
-    nb = nb + v[q - 1];
-    nb = nb + v[q + sy];
-    nb = nb + v[q - sy];
-    nb = nb + v[q + sz];
-    nb = nb + v[q - sz];
-    const float lap = (mu * (nb - 6.0f * c)) / (h * h);
-    p[d.at(x, y, z)] = r[q] - (lap - s[q] * c);
-}
-
-__device__ __forceinline__ float rz(const float* __restrict__ p, const Dims& d, int x, int y, int z) {
-    return (x < d.X && y < d.Y && z < d.Z) ? p[d.at(x, y, z)] : 0.0f;
+// A thread marches zc planes of one quad.  256^3 (134 MB): 27 us (5.0 TB/s), where
+// the whole-grid kernels took 57.
+template <int BLACK>
+__global__ void __launch_bounds__(256) k_gs_half(Trio v, Trio r, const float* __restrict__ s, Grid g, float mu, float h,
+                                                 int zc) {
+    int i, y;
+    if (!quad_of(g.xs, g.d.Y - 2, i, y)) return;
+    y += 1;
+    const int X = g.d.X, Y = g.d.Y, Z = g.d.Z;
+    const i64 sy = g.xs, sz = (i64)g.xs * Y;
+    const float* __restrict__ o = v.p[blockIdx.z] + (BLACK ? 0 : g.m);
+    float* __restrict__ w = v.p[blockIdx.z] + (BLACK ? g.m : 0);
+    const float* __restrict__ rr = r.p[blockIdx.z] + (BLACK ? g.m : 0);
+    const float* __restrict__ ss = s + (BLACK ? g.m : 0);
+    const int z0 = 1 + blockIdx.y * zc, z1 = min(Z - 1, z0 + zc);
+    float om[4], oc[4], op[4];
+    i64 q = g.row(y, z0) + i;
+    ld4a(om, o + q - sz);
+    ld4a(oc, o + q);
+    for (int z = z0; z < z1; z++, q += sz) {
+        const int e = ((y + z) & 1) ^ BLACK;  // the cells have x = 2 i + e
+        float yp[4], ym[4], r4[4], s4[4], val[4];
+        const float sc = o[q + (e ? 4 : -1)];
+        ld4a(op, o + q + sz);
+        ld4a(yp, o + q + sy);
+        ld4a(ym, o + q - sy);
+        ld4a(r4, rr + q);
+        ld4a(s4, ss + q);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float side = e ? (j < 3 ? oc[j + 1] : sc) : (j > 0 ? oc[j - 1] : sc);
+            float nb = oc[j] + side;
+            nb = nb + yp[j];
+            nb = nb + ym[j];
+            nb = nb + op[j];
+            nb = nb + om[j];
+            val[j] = gs_value(nb, r4[j], s4[j], mu, h);
+        }
+        if (i == 0 && e == 0) val[0] = val[1];  // x = 0
+        const int last = X - 1 - 2 * i - e;     // x = X - 1 is element last / 2
+        if (last == 0) {                        // its mirror is in the quad before
+            const i64 k = q - 1;
+            float nb = o[k] + o[k + (e ? 1 : -1)];
+            nb = nb + o[k + sy];
+            nb = nb + o[k - sy];
+            nb = nb + o[k + sz];
+            nb = nb + o[k - sz];
+            val[0] = gs_value(nb, rr[k], ss[k], mu, h);
+        }
+#pragma unroll
+        for (int j = 1; j < 4; j++)
+            if (last == 2 * j) val[j] = val[j - 1];
+        // this cell's row and plane, and the boundary rows and planes it mirrors
+        auto rows_of = [&](i64 k) {
+            st4a(w + k, val);
+            if (y == 2) st4a(w + k - 2 * sy, val);
+            if (y == Y - 3) st4a(w + k + 2 * sy, val);
+        };
+        rows_of(q);
+        if (z == 2) rows_of(q - 2 * sz);
+        if (z == Z - 3) rows_of(q + 2 * sz);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            om[j] = oc[j];
+            oc[j] = op[j];
+        }
+    }
 }
 
 // restrictVolume, kernels_no_3d_write.cl:2218-2246: 2x2x2 mean, zero outside.
-__global__ void k_restrict(const float* __restrict__ fine, Dims fd, Dims cd, float* __restrict__ coarse) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(cd, x, y)) return;
-    const int X = 2 * x, Y = 2 * y, Z = 2 * z;
-    float s = rz(fine, fd, X, Y, Z);
-    s = s + rz(fine, fd, X + 1, Y, Z);
-    s = s + rz(fine, fd, X, Y + 1, Z);
-    s = s + rz(fine, fd, X, Y, Z + 1);
-    s = s + rz(fine, fd, X + 1, Y + 1, Z);
-    s = s + rz(fine, fd, X, Y + 1, Z + 1);
-    s = s + rz(fine, fd, X + 1, Y + 1, Z + 1);
-    s = s + rz(fine, fd, X + 1, Y, Z + 1);
-    coarse[cd.at(x, y, z)] = 0.125f * s;
+// A thread makes four coarse cells of a row; `row8(y, z, i, ev, od)` gives the
+// eight fine values x = 2i .. 2i + 7 of a row.
+template <class R>
+__device__ __forceinline__ void restrict_quad(const Grid& f, const Grid& c, int i, int y, int z, float* out, R row8) {
+    float ev[2][2][4], od[2][2][4];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            const int Y = 2 * y + a, Z = 2 * z + b;
+            if (2 * i < f.d.X && Y < f.d.Y && Z < f.d.Z) {
+                row8(Y, Z, i, ev[a][b], od[a][b]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (2 * (i + j) >= f.d.X) ev[a][b][j] = 0.0f;
+                    if (2 * (i + j) + 1 >= f.d.X) od[a][b][j] = 0.0f;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) ev[a][b][j] = od[a][b][j] = 0.0f;
+            }
+        }
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float s = ev[0][0][j];
+        s = s + od[0][0][j];
+        s = s + ev[1][0][j];
+        s = s + ev[0][1][j];
+        s = s + od[1][0][j];
+        s = s + ev[1][1][j];
+        s = s + od[1][1][j];
+        s = s + od[0][1][j];
+        v[j] = 0.125f * s;
+    }
+    const int odd = (y + z) & 1;
+    float* o = out + c.row(y, z) + (i >> 1);
+    *reinterpret_cast<float2*>(o + (odd ? c.m : 0)) = make_float2(v[0], v[2]);
+    *reinterpret_cast<float2*>(o + (odd ? 0 : c.m)) = make_float2(v[1], v[3]);
 }
 
-// prolongate (ADD) / prolongate2, kernels_no_3d_write.cl:2248-2266: injection.
-template <bool ADD>
-__global__ void k_prolong(const float* __restrict__ coarse, Dims cd, Dims fd, float* v) {
-    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
-    if (!in_dims(fd, x, y)) return;
-    const float c = rz(coarse, cd, x / 2, y / 2, z / 2);
-    const i64 i = fd.at(x, y, z);
-    v[i] = ADD ? v[i] + c : c;
+__global__ void __launch_bounds__(256) k_restrict(Trio fine, Grid f, Grid c, Trio coarse) {
+    int i, y;
+    if (!quad_of(c.d.X, c.d.Y, i, y)) return;
+    const float* a = fine.p[blockIdx.z];
+    restrict_quad(f, c, i, y, blockIdx.y, coarse.p[blockIdx.z], [&](int Y, int Z, int k, float* ev, float* od) {
+        float t[4];
+        ld4a(t, even_x(f, a, Y, Z) + k);
+        __builtin_memcpy(ev, t, 16);
+        ld4a(t, odd_x(f, a, Y, Z) + k);
+        __builtin_memcpy(od, t, 16);
+    });
 }
 
-__global__ void k_add_inplace(float* __restrict__ f, const float* __restrict__ e, i64 n) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) f[i] = f[i] + e[i];
+// residual, kernels_no_3d_write.cl:2268-2301, restricted on the way.  (h h is
+// a power of four: the product with its reciprocal rounds as the quotient.)
+__device__ __forceinline__ float residual_of(float r, float s, float c, float nb, float mu, float ih2) {
+    const float lap = (mu * (nb - 6.0f * c)) * ih2;
+    return r - (lap - s * c);
+}
+__global__ void __launch_bounds__(256) k_residual_restrict(Trio v3, Trio r3, const float* __restrict__ s, Grid g,
+                                                           Grid cg, float mu, float ih2, Trio coarse) {
+    int i0, y0;
+    if (!quad_of(cg.d.X, cg.d.Y, i0, y0)) return;
+    const float *v = v3.p[blockIdx.z], *r = r3.p[blockIdx.z];
+    const int X = g.d.X;
+    restrict_quad(g, cg, i0, y0, blockIdx.y, coarse.p[blockIdx.z], [&](int Y, int Z, int i, float* ev, float* od) {
+        const int y = remap(Y, g.d.Y), z = remap(Z, g.d.Z);
+        const float *E = even_x(g, v, y, z) + i, *O = odd_x(g, v, y, z) + i;
+        float e[4], o[4], a[4], b[4], c[4], d[4], re[4], se[4];
+        ld4a(e, E);
+        ld4a(o, O);
+        ld4a(a, even_x(g, v, y + 1, z) + i);
+        ld4a(b, even_x(g, v, y - 1, z) + i);
+        ld4a(c, even_x(g, v, y, z + 1) + i);
+        ld4a(d, even_x(g, v, y, z - 1) + i);
+        ld4a(re, even_x(g, r, y, z) + i);
+        ld4a(se, even_x(g, s, y, z) + i);
+        const float before = O[-1], after = E[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float nb = o[j];
+            nb = nb + (j ? o[j - 1] : before);
+            nb = nb + a[j];
+            nb = nb + b[j];
+            nb = nb + c[j];
+            nb = nb + d[j];
+            ev[j] = residual_of(re[j], se[j], e[j], nb, mu, ih2);
+        }
+        ld4a(a, odd_x(g, v, y + 1, z) + i);
+        ld4a(b, odd_x(g, v, y - 1, z) + i);
+        ld4a(c, odd_x(g, v, y, z + 1) + i);
+        ld4a(d, odd_x(g, v, y, z - 1) + i);
+        ld4a(re, odd_x(g, r, y, z) + i);
+        ld4a(se, odd_x(g, s, y, z) + i);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float nb = j < 3 ? e[j + 1] : after;
+            nb = nb + e[j];
+            nb = nb + a[j];
+            nb = nb + b[j];
+            nb = nb + c[j];
+            nb = nb + d[j];
+            od[j] = residual_of(re[j], se[j], o[j], nb, mu, ih2);
+        }
+        if (i == 0) ev[0] = ev[1];     // x = 0
+        const int last = X - 1 - 2 * i;  // x = X - 1
+        if (last == 0 || last == 1) {  // its mirror X - 3 is in the quad before
+            const bool odd = last == 1;
+            const float *C = (odd ? O : E) - 1, *N = odd ? E : O;  // N: the row's other colour
+            const float* a4[4] = {odd ? odd_x(g, v, y + 1, z) : even_x(g, v, y + 1, z),
+                                  odd ? odd_x(g, v, y - 1, z) : even_x(g, v, y - 1, z),
+                                  odd ? odd_x(g, v, y, z + 1) : even_x(g, v, y, z + 1),
+                                  odd ? odd_x(g, v, y, z - 1) : even_x(g, v, y, z - 1)};
+            float nb = odd ? N[0] : N[-1];
+            nb = nb + (odd ? N[-1] : N[-2]);
+            for (int k = 0; k < 4; k++) nb = nb + a4[k][i - 1];
+            const float rv = (odd ? odd_x(g, r, y, z) : even_x(g, r, y, z))[i - 1];
+            const float sv = (odd ? odd_x(g, s, y, z) : even_x(g, s, y, z))[i - 1];
+            (odd ? od : ev)[0] = residual_of(rv, sv, C[0], nb, mu, ih2);
+        }
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            if (last == 2 * j) ev[j] = ev[j - 1];
+            if (last == 2 * j + 1) od[j] = od[j - 1];
+        }
+    });
 }
 
+// prolongate (ADD) / prolongate2, kernels_no_3d_write.cl:2248-2266: injection,
+// into the black cells and, with RED, the red ones.
+template <bool ADD, bool RED>
+__global__ void __launch_bounds__(256) k_prolong(Trio coarse, Grid c, Grid f, Trio fine) {
+    int i, y;
+    if (!quad_of(f.xs, f.d.Y, i, y)) return;
+    const int z = blockIdx.y;
+    // element i + j of either colour lies in coarse column i + j
+    const float2 e = *reinterpret_cast<const float2*>(even_x(c, coarse.p[blockIdx.z], y >> 1, z >> 1) + (i >> 1));
+    const float2 o = *reinterpret_cast<const float2*>(odd_x(c, coarse.p[blockIdx.z], y >> 1, z >> 1) + (i >> 1));
+    const float cv[4] = {e.x, o.x, e.y, o.y};
+#pragma unroll
+    for (int b = RED ? 0 : 1; b < 2; b++) {
+        float* p = fine.p[blockIdx.z] + f.row(y, z) + i + (b ? f.m : 0);
+        float v[4];
+        if (ADD) ld4a(v, p);
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = ADD ? v[j] + cv[j] : cv[j];
+        st4a(p, v);
+    }
+}
+
+// f += e on the finest grid; f is a plain array
+__global__ void __launch_bounds__(256) k_add_inplace(float* __restrict__ f, const float* __restrict__ e, Grid g) {
+    int i, y;
+    if (!quad_of(g.xs, g.d.Y, i, y)) return;
+    const int z = blockIdx.y;
+    float ev[4], od[4];
+    ld4a(ev, even_x(g, e, y, z) + i);
+    ld4a(od, odd_x(g, e, y, z) + i);
+    float* p = f + g.d.at(2 * i, y, z);
+    if (2 * i + 7 < g.d.X) {
+        float t[8];
+        __builtin_memcpy(t, p, 32);
+#pragma unroll
+        for (int j = 0; j < 8; j++) t[j] = t[j] + ((j & 1) ? od[j >> 1] : ev[j >> 1]);
+        __builtin_memcpy(p, t, 32);
+    } else {
+        for (int j = 0; j < 8; j++)
+            if (2 * i + j < g.d.X) p[j] = p[j] + ((j & 1) ? od[j >> 1] : ev[j >> 1]);
+    }
+}
+
+// n quads from element `from` of each array
+__global__ void __launch_bounds__(256) k_zero(Trio v, i64 from, i64 n) {
+    float4* p = reinterpret_cast<float4*>(v.p[blockIdx.z] + from);
+    for (i64 i = blockIdx.x * (i64)256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) p[i] = make_float4(0, 0, 0, 0);
+}
 __global__ void k_fill(float* __restrict__ p, i64 n, float v) {
     for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) p[i] = v;
 }
@@ -192,60 +462,101 @@ static Dims coarser(Dims d) {
 }
 
 struct Level {
-    Dims d;
-    float *r, *v, *s, *t, *p;
+    Grid g;
+    Trio r, v;
+    float* s;
 };
+
+// cells up to which a level runs its components in one launch
+constexpr i64 FMG_WIDE = (i64)1 << 22;
+// cells of the finest grid up to which all three components have buffers
+constexpr i64 FMG_TOGETHER = (i64)1 << 27;
 
 struct Solver {
     std::vector<Level> L;
     float mu;
     int v0, v1, v2;
+    int comps;  // components per cycle
     hipStream_t st;
     tsf_status err = TSF_OK;
 
     void chk() {
         if (err == TSF_OK) err = check_launch("tsf_gvf_fmg");
     }
-    void zero(float* p, Dims d) {
-        hipLaunchKernelGGL(k_fill, g1(d.n()), 256, 0, st, p, d.n(), 0.0f);
+    static Trio from(const Trio& t, int c) { return Trio{{t.p[c], t.p[c < 2 ? c + 1 : 2], t.p[2]}}; }
+    // f(c, n): n components from c, all in one launch or one by one
+    template <class F>
+    void split(int l, F f) {
+        if (L[l].g.d.n() <= FMG_WIDE) f(0, comps);
+        else
+            for (int c = 0; c < comps; c++) f(c, 1);
+    }
+    // v = 0: the black cells, and the red ones unless a sweep comes first
+    void zero(int l, int c, int n, bool red) {
+        const Grid& g = L[l].g;
+        const i64 cells = red ? 2 * g.m : g.m;
+        hipLaunchKernelGGL(k_zero, dim3(g1(cells / 4), 1, n), 256, 0, st, from(L[l].v, c), red ? 0 : g.m, cells / 4);
         chk();
     }
-    void smooth(int l, int iters) {
+    void smooth(int l, int c, int n, int iters) {
         Level& a = L[l];
         const float h = (float)(1 << l);
+        const int planes = a.g.d.Z - 2;
+        // planes per thread: the neighbour planes stay in registers, but 2048
+        // workgroups (8 per compute unit) come first
+        int zc = 8;
+        while (zc > 1 && (i64)quad_grid(a.g.xs, a.g.d.Y - 2, 1, n).x * n * ((planes + zc - 1) / zc) < 2048) zc /= 2;
+        const dim3 gr = quad_grid(a.g.xs, a.g.d.Y - 2, (planes + zc - 1) / zc, n);
         for (int i = 0; i < iters; i++) {
-            hipLaunchKernelGGL(k_gs_red, STENCIL_GRID(a.d), 0, st, a.v, a.r, a.s, a.d, mu, h, a.t);
-            hipLaunchKernelGGL(k_gs_black, STENCIL_GRID(a.d), 0, st, a.t, a.r, a.s, a.d, mu, h, a.v);
+            hipLaunchKernelGGL(k_gs_half<0>, gr, 256, 0, st, from(a.v, c), from(a.r, c), a.s, a.g, mu, h, zc);
+            hipLaunchKernelGGL(k_gs_half<1>, gr, 256, 0, st, from(a.v, c), from(a.r, c), a.s, a.g, mu, h, zc);
             chk();
         }
+    }
+    template <bool ADD>
+    void prolong(int l, int c, int n, bool red) {
+        Level &a = L[l], &b = L[l + 1];
+        const dim3 gr = quad_grid(a.g.xs, a.g.d.Y, a.g.d.Z, n);
+        if (red) hipLaunchKernelGGL((k_prolong<ADD, true>), gr, 256, 0, st, from(b.v, c), b.g, a.g, from(a.v, c));
+        else hipLaunchKernelGGL((k_prolong<ADD, false>), gr, 256, 0, st, from(b.v, c), b.g, a.g, from(a.v, c));
+        chk();
     }
     void vcycle(int l) {
-        Level& a = L[l];
-        smooth(l, v1);
-        if (l + 1 < (int)L.size()) {
+        const bool last = l + 1 == (int)L.size();
+        split(l, [&](int c, int n) {
+            Level& a = L[l];
+            smooth(l, c, n, v1);
+            if (last) {
+                smooth(l, c, n, v2);
+                return;
+            }
             Level& b = L[l + 1];
             const float h = (float)(1 << l);
-            hipLaunchKernelGGL(k_residual, STENCIL_GRID(a.d), 0, st, a.r, a.v, a.s, a.d, mu, h, a.p);
-            hipLaunchKernelGGL(k_restrict, STENCIL_GRID(b.d), 0, st, a.p, a.d, b.d, b.r);
+            hipLaunchKernelGGL(k_residual_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st, from(a.v, c),
+                               from(a.r, c), a.s, a.g, b.g, mu, 1.0f / (h * h), from(b.r, c));
             chk();
-            zero(b.v, b.d);
-            vcycle(l + 1);
-            hipLaunchKernelGGL(k_prolong<true>, STENCIL_GRID(a.d), 0, st, b.v, b.d, a.d, a.v);
-            chk();
-        }
-        smooth(l, v2);
+            zero(l + 1, c, n, v1 == 0);
+        });
+        if (last) return;
+        vcycle(l + 1);
+        split(l, [&](int c, int n) {
+            prolong<true>(l, c, n, v2 == 0);
+            smooth(l, c, n, v2);
+        });
     }
     void fmg(int l) {
-        Level& a = L[l];
+        const bool red = v0 == 0 || v1 == 0;
         if (l + 1 < (int)L.size()) {
-            Level& b = L[l + 1];
-            hipLaunchKernelGGL(k_restrict, STENCIL_GRID(b.d), 0, st, a.r, a.d, b.d, b.r);
-            chk();
+            split(l, [&](int c, int n) {
+                Level &a = L[l], &b = L[l + 1];
+                hipLaunchKernelGGL(k_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st, from(a.r, c), a.g,
+                                   b.g, from(b.r, c));
+                chk();
+            });
             fmg(l + 1);
-            hipLaunchKernelGGL(k_prolong<false>, STENCIL_GRID(a.d), 0, st, b.v, b.d, a.d, a.v);
-            chk();
+            split(l, [&](int c, int n) { prolong<false>(l, c, n, red); });
         } else {
-            zero(a.v, a.d);
+            split(l, [&](int c, int n) { zero(l, c, n, red); });
         }
         for (int i = 0; i < v0; i++) vcycle(l);
     }
@@ -257,6 +568,9 @@ static std::vector<Dims> level_dims(Dims d, int levels) {
     return v;
 }
 
+// a colour-split array of one grid
+static size_t array_bytes(const Grid& g) { return ((size_t)g.m * 8 + 255) & ~(size_t)255; }
+
 }  // namespace tsf
 
 using namespace tsf;
@@ -265,8 +579,9 @@ extern "C" {
 
 size_t tsf_gvf_fmg_workspace_size(tsf_dims dims, int32_t levels) {
     if (levels < 0 || levels > 12) return 0;
+    const size_t arrays = 2 * (D(dims).n() <= FMG_TOGETHER ? 3 : 1) + 1;  // r and v per component, s
     size_t b = 0;
-    for (Dims d : level_dims(D(dims), levels)) b += 5 * (((size_t)d.n() * 4 + 255) & ~(size_t)255);
+    for (Dims d : level_dims(D(dims), levels)) b += arrays * array_bytes(Grid(d));
     return b + NPART * sizeof(double) + 256;
 }
 
@@ -293,49 +608,63 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
     S.v0 = v0;
     S.v1 = v1;
     S.v2 = v2;
+    S.comps = D(dims).n() <= FMG_TOGETHER ? 3 : 1;
     S.st = stream;
     char* p = (char*)sc.ptr;
     for (Dims d : ld) {
-        size_t b = ((size_t)d.n() * 4 + 255) & ~(size_t)255;
-        Level lv;
-        lv.d = d;
-        float** bufs[5] = {&lv.r, &lv.v, &lv.s, &lv.t, &lv.p};
-        for (float** q : bufs) {
-            *q = (float*)p;
+        Level lv{Grid(d), {}, {}, nullptr};
+        const size_t b = array_bytes(lv.g);
+        auto next = [&] {
+            float* q = (float*)p;
             p += b;
+            return q;
+        };
+        for (int c = 0; c < 3; c++) {
+            lv.r.p[c] = c < S.comps ? next() : lv.r.p[0];
+            lv.v.p[c] = c < S.comps ? next() : lv.v.p[0];
         }
+        lv.s = next();
         S.L.push_back(lv);
     }
     double* part = (double*)p;
     double* norm_out = part + NPART;
-    const float *Fx = (const float*)f->x, *Fy = (const float*)f->y, *Fz = (const float*)f->z;
+    const float* F[3] = {(const float*)f->x, (const float*)f->y, (const float*)f->z};
     float* O[3] = {(float*)out->x, (float*)out->y, (float*)out->z};
-    const Dims d0 = ld[0];
-    const i64 n0 = d0.n();
+    const Grid g0 = S.L[0].g;
+    const i64 n0 = g0.d.n();
+    const dim3 gr0 = quad_grid(g0.xs, g0.d.Y, g0.d.Z, 1);
     // |F|^2 at every level (restricted once)
-    hipLaunchKernelGGL(k_sqrmag, g1(n0), 256, 0, stream, Fx, Fy, Fz, S.L[0].s, n0);
+    hipLaunchKernelGGL(k_sqrmag, gr0, 256, 0, stream, F[0], F[1], F[2], g0, S.L[0].s);
     S.chk();
-    for (size_t l = 1; l < S.L.size(); l++)
-        hipLaunchKernelGGL(k_restrict, STENCIL_GRID(S.L[l].d), 0, stream, S.L[l - 1].s, S.L[l - 1].d, S.L[l].d,
-                           S.L[l].s);
+    for (size_t l = 1; l < S.L.size(); l++) {
+        const Grid &a = S.L[l - 1].g, &b = S.L[l].g;
+        hipLaunchKernelGGL(k_restrict, quad_grid(b.d.X, b.d.Y, b.d.Z, 1), 256, 0, stream,
+                           Trio{{S.L[l - 1].s, nullptr, nullptr}}, a, b, Trio{{S.L[l].s, nullptr, nullptr}});
+    }
     S.chk();
-    for (int c = 0; c < 3 && S.err == TSF_OK; c++) {
-        S.zero(O[c], d0);
+    for (int c0 = 0; c0 < 3 && S.err == TSF_OK; c0 += S.comps) {
+        for (int k = 0; k < S.comps; k++)
+            hipLaunchKernelGGL(k_fill, g1(n0), 256, 0, stream, O[c0 + k], n0, 0.0f);
+        S.chk();
         for (int it = 0; it < iterations && S.err == TSF_OK; it++) {
-            hipLaunchKernelGGL(k_fmg_residual, STENCIL_GRID(d0), 0, stream, Fx, Fy, Fz, O[c], d0, mu, c, S.L[0].r);
-            S.chk();
-            if (residual_norms) {
-                hipLaunchKernelGGL(k_sumsq_partial, NPART, 256, 0, stream, S.L[0].r, n0, part);
-                hipLaunchKernelGGL(k_sum_partials, 1, 256, 0, stream, part, NPART, norm_out);
+            for (int k = 0; k < S.comps; k++) {
+                const int c = c0 + k;
+                hipLaunchKernelGGL(k_fmg_residual, gr0, 256, 0, stream, F[c], O[c], S.L[0].s, g0, mu, S.L[0].r.p[k]);
                 S.chk();
-                double ss = 0.0;
-                hipError_t e = hipMemcpyAsync(&ss, norm_out, sizeof ss, hipMemcpyDeviceToHost, stream);
-                if (e == hipSuccess) e = hipStreamSynchronize(stream);
-                if (e != hipSuccess) return set_error(TSF_ERR_HIP, "%s: %s", W, hipGetErrorString(e));
-                residual_norms[c * iterations + it] = sqrt(ss);
+                if (residual_norms) {
+                    hipLaunchKernelGGL(k_sumsq_partial, NPART, 256, 0, stream, S.L[0].r.p[k], 2 * g0.m, part);
+                    hipLaunchKernelGGL(k_sum_partials, 1, 256, 0, stream, part, NPART, norm_out);
+                    S.chk();
+                    double ss = 0.0;
+                    hipError_t e = hipMemcpyAsync(&ss, norm_out, sizeof ss, hipMemcpyDeviceToHost, stream);
+                    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+                    if (e != hipSuccess) return set_error(TSF_ERR_HIP, "%s: %s", W, hipGetErrorString(e));
+                    residual_norms[c * iterations + it] = sqrt(ss);
+                }
             }
             S.fmg(0);
-            hipLaunchKernelGGL(k_add_inplace, g1(n0), 256, 0, stream, O[c], S.L[0].v, n0);
+            for (int k = 0; k < S.comps; k++)
+                hipLaunchKernelGGL(k_add_inplace, gr0, 256, 0, stream, O[c0 + k], S.L[0].v.p[k], g0);
             S.chk();
         }
     }
