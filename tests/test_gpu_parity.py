@@ -391,6 +391,42 @@ def test_tdf_wide_halo(tsf, orc, mode):
     assert np.array_equal(r.download(), er)
 
 
+@pytest.mark.parametrize("storage", [0, 1, 2, 3])
+def test_tdf_gather_inside_and_at_the_faces(tsf, orc, storage):
+    """Gathered samples in bricks that radius after radius lose their room
+    inside the volume (unclamped taps, then clamped ones), every storage."""
+    shape = (44, 50, 90)
+    V = _gvf_field(orc, shape, 16)
+    fld = tsf.Field.from_host(V, storage, 1.0 if storage in (0, 3) else _f16_scale(V))
+    t, r = tsf.DeviceArray(shape, np.float32), tsf.DeviceArray(shape, np.float32)
+    tsf.tdf_circle(fld, 2.5, 18.0, 0.5, t, r)
+    et, er = orc.tdf_circle(fld.download(), 2.5, 18.0, 0.5, "f32")
+    assert np.isfinite(et).all() and (et > 0).sum() > 100
+    assert np.array_equal(t.download(), et) and np.array_equal(r.download(), er)
+
+
+def test_tdf_gather_wide_planes(tsf, orc):
+    """Planes of more than 2^24 texels gather through 64-bit addresses: the
+    corner of such a volume equals the same corner in a small one."""
+    small, big = (3, 96, 96), (3, 4097, 4096)
+    z, y, x = np.mgrid[:small[0], :small[1], :small[2]].astype(np.float32)
+    V = np.full((4,) + small, 0.01, np.float32)  # a tube along z; 0.01 everywhere past row and column 80
+    g = np.where((x < 80) & (y < 80), np.exp(-((x - 33) ** 2 + (y - 30) ** 2) / 50.0), 0.0) * (1 + 0.1 * z)
+    V[0] += (33 - x) * g / 8
+    V[1] += (30 - y) * g / 8
+    V[3] = np.sqrt((V[:3] ** 2).sum(0))
+    W = np.full((4,) + big, V[0, 0, 95, 95], np.float32)
+    W[3] = V[3, 0, 95, 95]
+    W[:, :, :96, :96] = V
+    got = []
+    for shape, F in ((small, V), (big, W)):
+        t, r = tsf.DeviceArray(shape, np.float32), tsf.DeviceArray(shape, np.float32)
+        tsf.tdf_circle(tsf.Field.from_host(F, 1, _f16_scale(V)), 2.5, 9.0, 0.5, t, r)
+        got.append((t.download()[:, :70, :70], r.download()[:, :70, :70]))
+    assert (got[0][0] > 0).sum() > 100
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("mode", ["f32", "f16", "mixed"])
 def test_tdf_deep_volume(tsf, orc, mode):
     """A volume 5600 planes deep, where the compile-time-stride kernels'

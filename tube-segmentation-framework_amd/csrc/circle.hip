@@ -70,6 +70,30 @@ __device__ __forceinline__ float circle_sum(const A& T, const Dims& d, float fx,
     return sum / 32.0f;
 }
 
+// The sample source of a brick that gathers: per circle, the unclamped taps
+// where no sample of the brick's voxels can leave the volume, the clamped
+// ones elsewhere.
+template <class S>
+struct BrickTex {
+    __amdgpu_buffer_rsrc_t b;
+    float inv;
+    int lo, hi_x, hi_y, hi_z;  // least voxel coordinate of the brick, room above its last voxel per axis
+};
+template <bool FUSED, class S>
+__device__ __forceinline__ float circle_sum(const BrickTex<S>& T, const Dims& d, float fx, float fy, float fz,
+                                            float radius, const float (&e2)[3], const float (&e3)[3],
+                                            const CircleTables& tab) {
+    // |r v| <= reach per axis for orthonormal e2, e3 (checked, with slack for
+    // the rounding); a sample's cell lies within 1.5 of its position
+    const float reach = fabsf(radius) * 1.001f + 1.75f;
+    bool in = reach <= (float)T.lo && reach <= (float)T.hi_x && reach <= (float)T.hi_y && reach <= (float)T.hi_z;
+#pragma unroll
+    for (int c = 0; c < 3; c++) in = in && e2[c] * e2[c] + e3[c] * e3[c] <= 1.0005f;
+    if (__ballot(!in) == 0)
+        return circle_sum<FUSED>(BufTex<S, true>{T.b, T.inv}, d, fx, fy, fz, radius, e2, e3, tab);
+    return circle_sum<FUSED>(BufTex<S, false>{T.b, T.inv}, d, fx, fy, fz, radius, e2, e3, tab);
+}
+
 // splineTDF (kernels_no_3d_write.cl:1574-1667) at one voxel, with the 12
 // arms runSplineTDF enqueues (tubeDetectionFilters.cpp:46): normalised
 // Hessian, eigenvectors e1..e3, and along each arm cos(a_j) e3 + sin(a_j) e2
@@ -329,18 +353,45 @@ __global__ void __launch_bounds__(BX* BY* BZ)
 // kernels (tdf_brick), so a wave runs as many radii as its voxels need and
 // not as many as its slowest voxel: only the compaction state is in LDS.
 // MIXED: the precision form's (Hessian from the F32 planes, fused samples).
-template <class S, bool NORM, bool MIXED, int BX, int BY, int BZ>
+// BUF: through a buffer resource of `bytes` (gather_buffer; bound by the
+// issue of a sample's instructions: 256 x 256 x 200, SNORM16, radii 2.5-15:
+// 7.1 ms with 64-bit tap addresses, 5.8 ms so, when the cache's
+// lookups, one per lane and load, bound it as much); larger arrays keep
+// the 64-bit addresses.
+template <class S, bool NORM, bool MIXED, bool BUF, int BX, int BY, int BZ>
 __global__ void __launch_bounds__(BX* BY* BZ)
-    k_tdf_gather(Tex<S> T, PlanesF32 H, Dims d, float rmin, float rmax, float rstep, CircleTables tab,
+    k_tdf_gather(Tex<S> T, unsigned bytes, PlanesF32 H, Dims d, float rmin, float rmax, float rstep, CircleTables tab,
                  float* __restrict__ tdf, float* __restrict__ rad) {
     int tbx, tby, tbz;
     xcd_tile(tbx, tby, tbz);
-    if constexpr (MIXED)
-        tdf_brick<NORM, BX, BY, BZ, true>(T, H, d, tbx * BX, tby * BY, tbz * BZ, rmin, rmax, rstep, tab, tdf, rad);
-    else
-        tdf_brick<NORM, BX, BY, BZ>(T, T, d, tbx * BX, tby * BY, tbz * BZ, rmin, rmax, rstep, tab, tdf, rad);
+    const int x = tbx * BX, y = tby * BY, z = tbz * BZ;
+    auto run = [&](const auto& src) {
+        if constexpr (MIXED) tdf_brick<NORM, BX, BY, BZ, true>(src, H, d, x, y, z, rmin, rmax, rstep, tab, tdf, rad);
+        else tdf_brick<NORM, BX, BY, BZ>(src, T, d, x, y, z, rmin, rmax, rstep, tab, tdf, rad);
+    };
+    if constexpr (BUF)
+        run(BrickTex<S>{__builtin_amdgcn_make_buffer_rsrc((void*)T.p, 0, (int)bytes, BUFFER_WORD3), T.inv,
+                        min(min(x, y), z), d.X - x - BX, d.Y - y - BY, d.Z - z - BZ});
+    else run(T);
 }
 constexpr int GBX = 16, GBY = 8, GBZ = 4;  // k_tdf_gather's bricks
+// Whether the texel array can be reached through BufTex's 32-bit offsets.
+static bool gather_buffer(Dims d, size_t texel) {
+    return (size_t)d.n() * texel < ((size_t)1 << 32) && (i64)d.X * d.Y < (1 << 24);
+}
+template <class S, bool NORM, bool MIXED>
+static void launch_gather(const void* tex, float inv, const PlanesF32& H, Dims d, float rmin, float rmax, float rstep,
+                          const CircleTables& tab, float* tdf, float* radius, hipStream_t stream) {
+    typedef typename Texel<S>::P P;
+    const dim3 grid((d.X + GBX - 1) / GBX, (d.Y + GBY - 1) / GBY, (d.Z + GBZ - 1) / GBZ), block(GBX, GBY, GBZ);
+    const Tex<S> T{(const P*)tex, inv};
+    if (gather_buffer(d, sizeof(P)))
+        hipLaunchKernelGGL((k_tdf_gather<S, NORM, MIXED, true, GBX, GBY, GBZ>), grid, block, 0, stream, T,
+                           (unsigned)(d.n() * sizeof(P)), H, d, rmin, rmax, rstep, tab, tdf, radius);
+    else
+        hipLaunchKernelGGL((k_tdf_gather<S, NORM, MIXED, false, GBX, GBY, GBZ>), grid, block, 0, stream, T, 0u, H, d,
+                           rmin, rmax, rstep, tab, tdf, radius);
+}
 
 // Stage the clamp-to-edge texels of a TX x TY x TZ tile at (ox, oy, oz) in
 // LDS, then a barrier: every load is issued before the first LDS store, so
@@ -664,9 +715,7 @@ static void launch_tdf(const void* tex, float inv, Dims d, float rmin, float rma
     // 256^3, radii 2.5-9 and 2.5-15: 15.2 -> 11.4 ms for F32 texels and
     // 14.7 -> 10.3 ms for SNORM16 against a per-voxel kernel without the
     // compaction)
-    const dim3 grid((d.X + GBX - 1) / GBX, (d.Y + GBY - 1) / GBY, (d.Z + GBZ - 1) / GBZ), block(GBX, GBY, GBZ);
-    hipLaunchKernelGGL((k_tdf_gather<S, NORM, false, GBX, GBY, GBZ>), grid, block, 0, stream,
-                       Tex<S>{(const P*)tex, inv}, PlanesF32{}, d, rmin, rmax, rstep, tab, tdf, radius);
+    launch_gather<S, NORM, false>(tex, inv, PlanesF32{}, d, rmin, rmax, rstep, tab, tdf, radius, stream);
 }
 
 // The compile-time-halo kernels on BX x BY x BZ bricks, when the float cell
@@ -699,9 +748,7 @@ static tsf_status launch_tdf_mixed(const tsf_field* f, const void* tex, float in
     const PlanesF32 H{(const float*)f->x, (const float*)f->y, (const float*)f->z, NORM ? (const float*)f->w : nullptr};
     if (h > 64 || lds + state > lds_per_block()) {
         (void)W;
-        const dim3 grid((d.X + GBX - 1) / GBX, (d.Y + GBY - 1) / GBY, (d.Z + GBZ - 1) / GBZ), block(GBX, GBY, GBZ);
-        hipLaunchKernelGGL((k_tdf_gather<S, NORM, true, GBX, GBY, GBZ>), grid, block, 0, stream,
-                           Tex<S>{(const P*)tex, inv}, H, d, rmin, rmax, rstep, tab, tdf, radius);
+        launch_gather<S, NORM, true>(tex, inv, H, d, rmin, rmax, rstep, tab, tdf, radius, stream);
         return TSF_OK;
     }
     // halos 4 and 5 (radii up to 3.5 and 4.5) with compile-time strides, on
