@@ -18,8 +18,9 @@
 // whole grids, every lane at work, in place.  The mirror of a boundary cell
 // (0 -> 2, N-1 -> N-3) has the cell's colour, so the boundary cells are
 // stored by the thread that computes their mirror.  A red half-sweep does not
-// read red cells, so what precedes one (zeroing, prolongation) sets the black
-// cells only.
+// read red cells, so what precedes one (zeroing, prolongation) is part of it;
+// the last half-sweep of a cycle adds to f, and both residuals are restricted
+// as they are made.
 //
 // The components do not depend on each other: grids up to 2^22 cells run all
 // three in one launch (a half-sweep of 64^3 cells takes 3 us for one and for
@@ -27,7 +28,11 @@
 // (201 MB at 256^3) can stay in the last-level cache.  Grids above 2^27 cells
 // keep one component's buffers only and run the cycles one after another.
 //
-// 256^3, two levels, 10 cycles: 27.7 ms on whole grids, 15.1 ms so.
+// 256^3, two levels, 10 cycles: 27.7 ms on whole grids, 15.1 ms split,
+// 13.1 ms with the zeroing, prolongation, restriction and f += e passes gone
+// into their neighbours.  Bound by the bytes of the finest grid (the
+// half-sweeps 24-28 us for 134 MB; two of them to a launch would have to read
+// the halo of both).
 #include <math.h>
 #include <vector>
 
@@ -81,13 +86,23 @@ __global__ void __launch_bounds__(256) k_sqrmag(const float* __restrict__ fx, co
     if (!quad_of(g.xs, g.d.Y, i, y)) return;
     const int z = blockIdx.y;
     const int odd = (y + z) & 1;
-    float e[2][4];
+    float e[2][4], a[8], b[8], c[8];
+    const i64 q = g.d.at(2 * i, y, z);
+    if (2 * i + 7 < g.d.X) {
+        __builtin_memcpy(a, fx + q, 32);
+        __builtin_memcpy(b, fy + q, 32);
+        __builtin_memcpy(c, fz + q, 32);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int x = 2 * i + j;
-        const i64 q = g.d.at(min(x, g.d.X - 1), y, z);
-        e[j & 1][j >> 1] = x < g.d.X ? fx[q] * fx[q] + fy[q] * fy[q] + fz[q] * fz[q] : 0.0f;
+        for (int j = 0; j < 8; j++) {
+            const bool in = 2 * i + j < g.d.X;
+            a[j] = in ? fx[q + j] : 0.0f;
+            b[j] = in ? fy[q + j] : 0.0f;
+            c[j] = in ? fz[q + j] : 0.0f;
+        }
     }
+#pragma unroll
+    for (int j = 0; j < 8; j++) e[j & 1][j >> 1] = a[j] * a[j] + b[j] * b[j] + c[j] * c[j];
     float* o = s + g.row(y, z) + i;
     st4a(o + (odd ? g.m : 0), e[0]);
     st4a(o + (odd ? 0 : g.m), e[1]);
@@ -99,25 +114,13 @@ __device__ __forceinline__ float fmg_residual_of(float fc, float c, float sq, fl
     const float residue = mu * (nb - 6.0f * c);
     return -sq * fc - (residue - sq * c);
 }
-__global__ void __launch_bounds__(256) k_fmg_residual(const float* __restrict__ Fc, const float* __restrict__ f,
-                                                      const float* __restrict__ s, Grid g, float mu,
-                                                      float* __restrict__ r) {
-    int i, y;
-    if (!quad_of(g.xs, g.d.Y, i, y)) return;
-    const int z = blockIdx.y, X = g.d.X;
+// the residuals x = 2 i .. 2 i + 7 of row (y, z), also stored in r
+__device__ __forceinline__ void fmg_residual_row(const float* __restrict__ Fc, const float* __restrict__ f,
+                                                 const float* __restrict__ s, const Grid& g, float mu, int y, int z,
+                                                 int i, float* __restrict__ r, float* ev, float* od) {
+    const int X = g.d.X;
     const int py = remap(y, g.d.Y), pz = remap(z, g.d.Z);
     const i64 sy = X, sz = (i64)X * g.d.Y, q = g.d.at(2 * i, py, pz);  // rows py, pz are interior: q - 1 .. q + 8 exist
-    auto at = [&](int x) {  // the value at column x, read apart
-        const i64 k = g.d.at(x, py, pz);
-        float nb = f[k + 1];
-        nb = nb + f[k - 1];
-        nb = nb + f[k + sy];
-        nb = nb + f[k - sy];
-        nb = nb + f[k + sz];
-        nb = nb + f[k - sz];
-        const float* sr = (x & 1) ? odd_x(g, s, py, pz) : even_x(g, s, py, pz);
-        return fmg_residual_of(Fc[k], f[k], sr[x >> 1], nb, mu);
-    };
     float e[2][4];
     if (2 * i + 7 < X) {
         float c[10], yp[8], ym[8], zp[8], zm[8], fc[8], se[4], so[4];
@@ -144,12 +147,40 @@ __global__ void __launch_bounds__(256) k_fmg_residual(const float* __restrict__ 
         if (i == 0) e[0][0] = e[0][1];
         if (2 * i + 7 == X - 1) e[1][3] = e[1][2];
     } else {
-        for (int j = 0; j < 8; j++) e[j & 1][j >> 1] = 2 * i + j < X ? at(remap(2 * i + j, X)) : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            float v = 0.0f;
+            if (2 * i + j < X) {
+                const int x = remap(2 * i + j, X);
+                const i64 k = g.d.at(x, py, pz);
+                float nb = f[k + 1];
+                nb = nb + f[k - 1];
+                nb = nb + f[k + sy];
+                nb = nb + f[k - sy];
+                nb = nb + f[k + sz];
+                nb = nb + f[k - sz];
+                const float* sr = (x & 1) ? odd_x(g, s, py, pz) : even_x(g, s, py, pz);
+                v = fmg_residual_of(Fc[k], f[k], sr[x >> 1], nb, mu);
+            }
+            e[j & 1][j >> 1] = v;
+        }
     }
     const int odd = (y + z) & 1;
     float* o = r + g.row(y, z) + i;
     st4a(o + (odd ? g.m : 0), e[0]);
     st4a(o + (odd ? 0 : g.m), e[1]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        ev[j] = e[0][j];
+        od[j] = e[1][j];
+    }
+}
+__global__ void __launch_bounds__(256) k_fmg_residual(const float* __restrict__ Fc, const float* __restrict__ f,
+                                                      const float* __restrict__ s, Grid g, float mu,
+                                                      float* __restrict__ r) {
+    int i, y;
+    float ev[4], od[4];
+    if (quad_of(g.xs, g.d.Y, i, y)) fmg_residual_row(Fc, f, s, g, mu, y, blockIdx.y, i, r, ev, od);
 }
 
 // GVFgaussSeidel / GVFgaussSeidel2 (the half-sweeps), kernels_no_3d_write.cl:
@@ -159,32 +190,80 @@ __device__ __forceinline__ float gs_value(float nb, float r, float s, float mu, 
     const float den = 12.0f * mu + h * h * s;
     return num / den;
 }
+// Where a red half-sweep takes the black cells from: the grid, the injected
+// coarse grid (prolongate2, kernels_no_3d_write.cl:2248-2266), the grid plus
+// that (prolongate), or nowhere (zeros).
+enum { FROM_GRID, FROM_COARSE, FROM_SUM, FROM_ZERO };
+struct HalfArgs {
+    Trio v, r;
+    const float* s;
+    Grid g;
+    float mu, h;
+    int zc;
+    Trio c;  // FROM_COARSE, FROM_SUM: the coarse grid
+    Grid cg;
+    Trio f;  // ADD: plain arrays
+};
+template <int FROM>
+struct Other {
+    const float* o;  // the other colour's cells
+    const float* c;
+    const HalfArgs& a;
+    // four elements from i (a multiple of 4) / element i of row (y, z); i = -1
+    // and i = the row length stand beside cells that a mirror replaces
+    __device__ __forceinline__ void quad(float (&v)[4], int y, int z, int i) const {
+        if (FROM == FROM_GRID || FROM == FROM_SUM) ld4a(v, o + a.g.row(y, z) + i);
+        if (FROM == FROM_ZERO) v[0] = v[1] = v[2] = v[3] = 0.0f;
+        if (FROM == FROM_COARSE || FROM == FROM_SUM) {
+            // element i + j of either colour lies in coarse column i + j
+            const float2 e = *reinterpret_cast<const float2*>(even_x(a.cg, c, y >> 1, z >> 1) + (i >> 1));
+            const float2 d = *reinterpret_cast<const float2*>(odd_x(a.cg, c, y >> 1, z >> 1) + (i >> 1));
+            const float cv[4] = {e.x, d.x, e.y, d.y};
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = FROM == FROM_SUM ? v[j] + cv[j] : cv[j];
+        }
+    }
+    __device__ __forceinline__ float one(int y, int z, int i) const {
+        float v = 0.0f;
+        if (FROM == FROM_GRID || FROM == FROM_SUM) v = o[a.g.row(y, z) + i];
+        if (FROM == FROM_COARSE || FROM == FROM_SUM) {
+            const int k = clampi(i, 0, a.g.xs - 1);
+            const float cv = ((k & 1) ? odd_x(a.cg, c, y >> 1, z >> 1) : even_x(a.cg, c, y >> 1, z >> 1))[k >> 1];
+            v = FROM == FROM_SUM ? v + cv : cv;
+        }
+        return v;
+    }
+};
+
 // A thread marches zc planes of one quad.  256^3 (134 MB): 27 us (5.0 TB/s), where
 // the whole-grid kernels took 57.
-template <int BLACK>
-__global__ void __launch_bounds__(256) k_gs_half(Trio v, Trio r, const float* __restrict__ s, Grid g, float mu, float h,
-                                                 int zc) {
+// ADD: the last half-sweep of a cycle on the finest grid: f += v, and v itself
+// is not stored.
+template <int BLACK, int FROM, bool ADD>
+__global__ void __launch_bounds__(256) k_gs_half(HalfArgs a) {
     int i, y;
+    const Grid g = a.g;
     if (!quad_of(g.xs, g.d.Y - 2, i, y)) return;
     y += 1;
     const int X = g.d.X, Y = g.d.Y, Z = g.d.Z;
-    const i64 sy = g.xs, sz = (i64)g.xs * Y;
-    const float* __restrict__ o = v.p[blockIdx.z] + (BLACK ? 0 : g.m);
-    float* __restrict__ w = v.p[blockIdx.z] + (BLACK ? g.m : 0);
-    const float* __restrict__ rr = r.p[blockIdx.z] + (BLACK ? g.m : 0);
-    const float* __restrict__ ss = s + (BLACK ? g.m : 0);
-    const int z0 = 1 + blockIdx.y * zc, z1 = min(Z - 1, z0 + zc);
+    const i64 sz = (i64)g.xs * Y;
+    float* const v = a.v.p[blockIdx.z];
+    const Other<FROM> o{v + (BLACK ? 0 : g.m), a.c.p[blockIdx.z], a};
+    float* __restrict__ w = v + (BLACK ? g.m : 0);
+    const float* __restrict__ rr = a.r.p[blockIdx.z] + (BLACK ? g.m : 0);
+    const float* __restrict__ ss = a.s + (BLACK ? g.m : 0);
+    const int z0 = 1 + blockIdx.y * a.zc, z1 = min(Z - 1, z0 + a.zc);
     float om[4], oc[4], op[4];
     i64 q = g.row(y, z0) + i;
-    ld4a(om, o + q - sz);
-    ld4a(oc, o + q);
+    o.quad(om, y, z0 - 1, i);
+    o.quad(oc, y, z0, i);
     for (int z = z0; z < z1; z++, q += sz) {
         const int e = ((y + z) & 1) ^ BLACK;  // the cells have x = 2 i + e
         float yp[4], ym[4], r4[4], s4[4], val[4];
-        const float sc = o[q + (e ? 4 : -1)];
-        ld4a(op, o + q + sz);
-        ld4a(yp, o + q + sy);
-        ld4a(ym, o + q - sy);
+        const float sc = o.one(y, z, e ? i + 4 : i - 1);
+        o.quad(op, y, z + 1, i);
+        o.quad(yp, y + 1, z, i);
+        o.quad(ym, y - 1, z, i);
         ld4a(r4, rr + q);
         ld4a(s4, ss + q);
 #pragma unroll
@@ -195,31 +274,48 @@ __global__ void __launch_bounds__(256) k_gs_half(Trio v, Trio r, const float* __
             nb = nb + ym[j];
             nb = nb + op[j];
             nb = nb + om[j];
-            val[j] = gs_value(nb, r4[j], s4[j], mu, h);
+            val[j] = gs_value(nb, r4[j], s4[j], a.mu, a.h);
         }
         if (i == 0 && e == 0) val[0] = val[1];  // x = 0
         const int last = X - 1 - 2 * i - e;     // x = X - 1 is element last / 2
         if (last == 0) {                        // its mirror is in the quad before
-            const i64 k = q - 1;
-            float nb = o[k] + o[k + (e ? 1 : -1)];
-            nb = nb + o[k + sy];
-            nb = nb + o[k - sy];
-            nb = nb + o[k + sz];
-            nb = nb + o[k - sz];
-            val[0] = gs_value(nb, rr[k], ss[k], mu, h);
+            float nb = o.one(y, z, i - 1) + o.one(y, z, e ? i : i - 2);
+            nb = nb + o.one(y + 1, z, i - 1);
+            nb = nb + o.one(y - 1, z, i - 1);
+            nb = nb + o.one(y, z + 1, i - 1);
+            nb = nb + o.one(y, z - 1, i - 1);
+            val[0] = gs_value(nb, rr[q - 1], ss[q - 1], a.mu, a.h);
         }
 #pragma unroll
         for (int j = 1; j < 4; j++)
             if (last == 2 * j) val[j] = val[j - 1];
         // this cell's row and plane, and the boundary rows and planes it mirrors
-        auto rows_of = [&](i64 k) {
-            st4a(w + k, val);
-            if (y == 2) st4a(w + k - 2 * sy, val);
-            if (y == Y - 3) st4a(w + k + 2 * sy, val);
+        auto put = [&](int py, int pz) {
+            if (!ADD) {
+                st4a(w + g.row(py, pz) + i, val);
+                return;
+            }
+            float* p = a.f.p[blockIdx.z] + g.d.at(2 * i, py, pz);
+            float t[8];
+            const bool whole = 2 * i + 7 < X;
+            if (whole) __builtin_memcpy(t, p, 32);
+            else
+                for (int j = 0; j < 8; j++) t[j] = 2 * i + j < X ? p[j] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) t[j] = t[j] + (((j ^ e) & 1) ? oc[j >> 1] : val[j >> 1]);
+            if (whole) __builtin_memcpy(p, t, 32);
+            else
+                for (int j = 0; j < 8; j++)
+                    if (2 * i + j < X) p[j] = t[j];
         };
-        rows_of(q);
-        if (z == 2) rows_of(q - 2 * sz);
-        if (z == Z - 3) rows_of(q + 2 * sz);
+        auto rows_of = [&](int pz) {
+            put(y, pz);
+            if (y == 2) put(0, pz);
+            if (y == Y - 3) put(Y - 1, pz);
+        };
+        rows_of(z);
+        if (z == 2) rows_of(0);
+        if (z == Z - 3) rows_of(Z - 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             om[j] = oc[j];
@@ -280,6 +376,19 @@ __global__ void __launch_bounds__(256) k_restrict(Trio fine, Grid f, Grid c, Tri
         __builtin_memcpy(ev, t, 16);
         ld4a(t, odd_x(f, a, Y, Z) + k);
         __builtin_memcpy(od, t, 16);
+    });
+}
+
+// k_fmg_residual, restricted on the way.
+__global__ void __launch_bounds__(256) k_fmg_residual_restrict(const float* __restrict__ Fc,
+                                                               const float* __restrict__ f,
+                                                               const float* __restrict__ s, Grid g, float mu,
+                                                               float* __restrict__ r, Grid cg,
+                                                               float* __restrict__ coarse) {
+    int i, y;
+    if (!quad_of(cg.d.X, cg.d.Y, i, y)) return;
+    restrict_quad(g, cg, i, y, blockIdx.y, coarse, [&](int Y, int Z, int k, float* ev, float* od) {
+        fmg_residual_row(Fc, f, s, g, mu, Y, Z, k, r, ev, od);
     });
 }
 
@@ -358,19 +467,17 @@ __global__ void __launch_bounds__(256) k_residual_restrict(Trio v3, Trio r3, con
     });
 }
 
-// prolongate (ADD) / prolongate2, kernels_no_3d_write.cl:2248-2266: injection,
-// into the black cells and, with RED, the red ones.
-template <bool ADD, bool RED>
+// prolongate (ADD) / prolongate2 where no sweep follows.
+template <bool ADD>
 __global__ void __launch_bounds__(256) k_prolong(Trio coarse, Grid c, Grid f, Trio fine) {
     int i, y;
     if (!quad_of(f.xs, f.d.Y, i, y)) return;
     const int z = blockIdx.y;
-    // element i + j of either colour lies in coarse column i + j
     const float2 e = *reinterpret_cast<const float2*>(even_x(c, coarse.p[blockIdx.z], y >> 1, z >> 1) + (i >> 1));
     const float2 o = *reinterpret_cast<const float2*>(odd_x(c, coarse.p[blockIdx.z], y >> 1, z >> 1) + (i >> 1));
     const float cv[4] = {e.x, o.x, e.y, o.y};
 #pragma unroll
-    for (int b = RED ? 0 : 1; b < 2; b++) {
+    for (int b = 0; b < 2; b++) {
         float* p = fine.p[blockIdx.z] + f.row(y, z) + i + (b ? f.m : 0);
         float v[4];
         if (ADD) ld4a(v, p);
@@ -380,7 +487,7 @@ __global__ void __launch_bounds__(256) k_prolong(Trio coarse, Grid c, Grid f, Tr
     }
 }
 
-// f += e on the finest grid; f is a plain array
+// f += e on the finest grid where no sweep ends a cycle; f is a plain array
 __global__ void __launch_bounds__(256) k_add_inplace(float* __restrict__ f, const float* __restrict__ e, Grid g) {
     int i, y;
     if (!quad_of(g.xs, g.d.Y, i, y)) return;
@@ -401,9 +508,9 @@ __global__ void __launch_bounds__(256) k_add_inplace(float* __restrict__ f, cons
     }
 }
 
-// n quads from element `from` of each array
-__global__ void __launch_bounds__(256) k_zero(Trio v, i64 from, i64 n) {
-    float4* p = reinterpret_cast<float4*>(v.p[blockIdx.z] + from);
+// n quads of each array
+__global__ void __launch_bounds__(256) k_zero(Trio v, i64 n) {
+    float4* p = reinterpret_cast<float4*>(v.p[blockIdx.z]);
     for (i64 i = blockIdx.x * (i64)256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) p[i] = make_float4(0, 0, 0, 0);
 }
 __global__ void k_fill(float* __restrict__ p, i64 n, float v) {
@@ -477,6 +584,7 @@ struct Solver {
     float mu;
     int v0, v1, v2;
     int comps;  // components per cycle
+    Trio f;     // and their f
     hipStream_t st;
     tsf_status err = TSF_OK;
 
@@ -491,74 +599,89 @@ struct Solver {
         else
             for (int c = 0; c < comps; c++) f(c, 1);
     }
-    // v = 0: the black cells, and the red ones unless a sweep comes first
-    void zero(int l, int c, int n, bool red) {
-        const Grid& g = L[l].g;
-        const i64 cells = red ? 2 * g.m : g.m;
-        hipLaunchKernelGGL(k_zero, dim3(g1(cells / 4), 1, n), 256, 0, st, from(L[l].v, c), red ? 0 : g.m, cells / 4);
+    // v as `from` says, where no sweep follows
+    void set(int l, int c, int n, int from) {
+        Level& a = L[l];
+        if (from == FROM_ZERO) {
+            const i64 quads = 2 * a.g.m / 4;
+            hipLaunchKernelGGL(k_zero, dim3(g1(quads), 1, n), 256, 0, st, Solver::from(a.v, c), quads);
+        } else if (from != FROM_GRID) {
+            Level& b = L[l + 1];
+            const dim3 gr = quad_grid(a.g.xs, a.g.d.Y, a.g.d.Z, n);
+            const Trio cv = Solver::from(b.v, c), fv = Solver::from(a.v, c);
+            if (from == FROM_SUM) hipLaunchKernelGGL(k_prolong<true>, gr, 256, 0, st, cv, b.g, a.g, fv);
+            else hipLaunchKernelGGL(k_prolong<false>, gr, 256, 0, st, cv, b.g, a.g, fv);
+        }
         chk();
     }
-    void smooth(int l, int c, int n, int iters) {
-        Level& a = L[l];
-        const float h = (float)(1 << l);
+    // sweeps on v, which starts as `from` says; add: the last one ends in f += v
+    void smooth(int l, int c, int n, int iters, int from, bool add) {
+        if (iters == 0) {
+            set(l, c, n, from);
+            if (add)
+                for (int k = c; k < c + n; k++)
+                    hipLaunchKernelGGL(k_add_inplace, quad_grid(L[0].g.xs, L[0].g.d.Y, L[0].g.d.Z, 1), 256, 0, st, f.p[k],
+                                       L[0].v.p[k], L[0].g);
+            chk();
+            return;
+        }
+        Level &a = L[l], &b = L[l + 1 < (int)L.size() ? l + 1 : l];
         const int planes = a.g.d.Z - 2;
         // planes per thread: the neighbour planes stay in registers, but 2048
         // workgroups (8 per compute unit) come first
         int zc = 8;
         while (zc > 1 && (i64)quad_grid(a.g.xs, a.g.d.Y - 2, 1, n).x * n * ((planes + zc - 1) / zc) < 2048) zc /= 2;
         const dim3 gr = quad_grid(a.g.xs, a.g.d.Y - 2, (planes + zc - 1) / zc, n);
+        const HalfArgs h{Solver::from(a.v, c), Solver::from(a.r, c), a.s, a.g, mu, (float)(1 << l), zc,
+                         Solver::from(b.v, c), b.g, Solver::from(f, c)};
         for (int i = 0; i < iters; i++) {
-            hipLaunchKernelGGL(k_gs_half<0>, gr, 256, 0, st, from(a.v, c), from(a.r, c), a.s, a.g, mu, h, zc);
-            hipLaunchKernelGGL(k_gs_half<1>, gr, 256, 0, st, from(a.v, c), from(a.r, c), a.s, a.g, mu, h, zc);
+            switch (i == 0 ? from : FROM_GRID) {
+                case FROM_GRID: hipLaunchKernelGGL((k_gs_half<0, FROM_GRID, false>), gr, 256, 0, st, h); break;
+                case FROM_COARSE: hipLaunchKernelGGL((k_gs_half<0, FROM_COARSE, false>), gr, 256, 0, st, h); break;
+                case FROM_SUM: hipLaunchKernelGGL((k_gs_half<0, FROM_SUM, false>), gr, 256, 0, st, h); break;
+                default: hipLaunchKernelGGL((k_gs_half<0, FROM_ZERO, false>), gr, 256, 0, st, h);
+            }
+            if (add && i + 1 == iters) hipLaunchKernelGGL((k_gs_half<1, FROM_GRID, true>), gr, 256, 0, st, h);
+            else hipLaunchKernelGGL((k_gs_half<1, FROM_GRID, false>), gr, 256, 0, st, h);
             chk();
         }
     }
-    template <bool ADD>
-    void prolong(int l, int c, int n, bool red) {
-        Level &a = L[l], &b = L[l + 1];
-        const dim3 gr = quad_grid(a.g.xs, a.g.d.Y, a.g.d.Z, n);
-        if (red) hipLaunchKernelGGL((k_prolong<ADD, true>), gr, 256, 0, st, from(b.v, c), b.g, a.g, from(a.v, c));
-        else hipLaunchKernelGGL((k_prolong<ADD, false>), gr, 256, 0, st, from(b.v, c), b.g, a.g, from(a.v, c));
-        chk();
-    }
-    void vcycle(int l) {
+    void vcycle(int l, int from, bool add) {
         const bool last = l + 1 == (int)L.size();
         split(l, [&](int c, int n) {
             Level& a = L[l];
-            smooth(l, c, n, v1);
+            smooth(l, c, n, v1, from, false);
             if (last) {
-                smooth(l, c, n, v2);
+                smooth(l, c, n, v2, FROM_GRID, add);
                 return;
             }
             Level& b = L[l + 1];
             const float h = (float)(1 << l);
-            hipLaunchKernelGGL(k_residual_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st, from(a.v, c),
-                               from(a.r, c), a.s, a.g, b.g, mu, 1.0f / (h * h), from(b.r, c));
+            hipLaunchKernelGGL(k_residual_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st,
+                               Solver::from(a.v, c), Solver::from(a.r, c), a.s, a.g, b.g, mu, 1.0f / (h * h),
+                               Solver::from(b.r, c));
             chk();
-            zero(l + 1, c, n, v1 == 0);
         });
         if (last) return;
-        vcycle(l + 1);
-        split(l, [&](int c, int n) {
-            prolong<true>(l, c, n, v2 == 0);
-            smooth(l, c, n, v2);
-        });
+        vcycle(l + 1, FROM_ZERO, false);
+        split(l, [&](int c, int n) { smooth(l, c, n, v2, FROM_SUM, add); });
     }
+    // level l from its r; on level 0, whose r is restricted already, f += v
     void fmg(int l) {
-        const bool red = v0 == 0 || v1 == 0;
+        int from = FROM_ZERO;
         if (l + 1 < (int)L.size()) {
-            split(l, [&](int c, int n) {
-                Level &a = L[l], &b = L[l + 1];
-                hipLaunchKernelGGL(k_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st, from(a.r, c), a.g,
-                                   b.g, from(b.r, c));
-                chk();
-            });
+            if (l > 0)
+                split(l, [&](int c, int n) {
+                    Level &a = L[l], &b = L[l + 1];
+                    hipLaunchKernelGGL(k_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, n), 256, 0, st,
+                                       Solver::from(a.r, c), a.g, b.g, Solver::from(b.r, c));
+                    chk();
+                });
             fmg(l + 1);
-            split(l, [&](int c, int n) { prolong<false>(l, c, n, red); });
-        } else {
-            split(l, [&](int c, int n) { zero(l, c, n, red); });
+            from = FROM_COARSE;
         }
-        for (int i = 0; i < v0; i++) vcycle(l);
+        for (int i = 0; i < v0; i++) vcycle(l, i == 0 ? from : FROM_GRID, l == 0 && i + 1 == v0);
+        if (v0 == 0) split(l, [&](int c, int n) { smooth(l, c, n, 0, from, l == 0); });
     }
 };
 
@@ -649,7 +772,15 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
         for (int it = 0; it < iterations && S.err == TSF_OK; it++) {
             for (int k = 0; k < S.comps; k++) {
                 const int c = c0 + k;
-                hipLaunchKernelGGL(k_fmg_residual, gr0, 256, 0, stream, F[c], O[c], S.L[0].s, g0, mu, S.L[0].r.p[k]);
+                S.f.p[k] = O[c];
+                if (S.L.size() > 1) {
+                    const Level& b = S.L[1];
+                    hipLaunchKernelGGL(k_fmg_residual_restrict, quad_grid(b.g.d.X, b.g.d.Y, b.g.d.Z, 1), 256, 0, stream,
+                                       F[c], O[c], S.L[0].s, g0, mu, S.L[0].r.p[k], b.g, b.r.p[k]);
+                } else {
+                    hipLaunchKernelGGL(k_fmg_residual, gr0, 256, 0, stream, F[c], O[c], S.L[0].s, g0, mu,
+                                       S.L[0].r.p[k]);
+                }
                 S.chk();
                 if (residual_norms) {
                     hipLaunchKernelGGL(k_sumsq_partial, NPART, 256, 0, stream, S.L[0].r.p[k], 2 * g0.m, part);
@@ -663,9 +794,6 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
                 }
             }
             S.fmg(0);
-            for (int k = 0; k < S.comps; k++)
-                hipLaunchKernelGGL(k_add_inplace, gr0, 256, 0, stream, O[c0 + k], S.L[0].v.p[k], g0);
-            S.chk();
         }
     }
     if (S.err != TSF_OK) return S.err;
