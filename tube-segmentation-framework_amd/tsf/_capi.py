@@ -377,10 +377,11 @@ CROP_THRESHOLD, CROP_LUNG = 0, 1
 def crop_scan_lines(src, method, threshold=0.0, stream=None):
     """Scan-line counts (lines_x, lines_y, lines_z) as int32 numpy arrays."""
     Z, Y, X = src.shape
-    lx, ly, lz = DeviceArray((X,), np.int32), DeviceArray((Y,), np.int32), DeviceArray((Z,), np.int32)
+    lines = DeviceArray((X + Y + Z,), np.int32)  # one allocation, one copy back
     _check(lib().tsf_crop_scan_lines(src.ptr, _TYPE_CODES[src.dtype], _dims(src.shape), int(method), threshold,
-                                     lx.ptr, ly.ptr, lz.ptr, _sp(stream)))
-    return lx.download(stream), ly.download(stream), lz.download(stream)
+                                     lines.ptr, lines.ptr + 4 * X, lines.ptr + 4 * (X + Y), _sp(stream)))
+    h = lines.download(stream)
+    return h[:X].copy(), h[X:X + Y].copy(), h[X + Y:].copy()
 
 
 def crop_region(lines_x, lines_y, lines_z, min_scan_lines, start_z_middle):
