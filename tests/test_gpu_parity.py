@@ -289,6 +289,20 @@ def test_gvf_fmg_shapes_and_sweeps(tsf, orc, shape, levels, sweeps):
     assert np.array_equal(out.download(), exp)
 
 
+def test_gvf_fmg_small_workspace(tsf, orc):
+    """A workspace of five grids per level (short of three components') runs
+    the components one by one; one below a component's is refused."""
+    shape, levels = (20, 22, 40), 2
+    F = _field_from(orc, phantom(shape, 11), fmax=0.2)
+    f, out = tsf.Field.from_host(F), tsf.Field(shape)
+    n = 5 * 4 * (20 * 22 * 40 + 32 ** 3 + 16 ** 3) + 10000
+    assert n < tsf.gvf_fmg_workspace_size(shape, levels)
+    tsf.gvf_fmg(f, out, 0.15, 2, levels, workspace=tsf.DeviceArray((n,), np.uint8))
+    assert np.array_equal(out.download(), orc.gvf_fmg(F, 0.15, 2, 1, 2, 2, levels, "f32"))
+    with pytest.raises(tsf.TSFError):
+        tsf.gvf_fmg(f, out, 0.15, 2, levels, workspace=tsf.DeviceArray((n // 2,), np.uint8))
+
+
 def test_gvf_fmg_one_component_at_a_time(tsf):
     """Above 2^27 cells the components share one set of buffers: what one
     leaves there must not reach the next, so permuted components (with a zero

@@ -26,7 +26,8 @@
 // three in one launch (a half-sweep of 64^3 cells takes 3 us for one and for
 // three), larger ones a component at a time, so that a phase's r, v and s
 // (201 MB at 256^3) can stay in the last-level cache.  Grids above 2^27 cells
-// keep one component's buffers only and run the cycles one after another.
+// keep one component's buffers only and run the cycles one after another, as
+// do smaller ones in a workspace that holds no more.
 //
 // 256^3, two levels, 10 cycles: 27.7 ms on whole grids, 15.1 ms split,
 // 13.1 ms with the zeroing, prolongation, restriction and f += e passes gone
@@ -693,6 +694,12 @@ static std::vector<Dims> level_dims(Dims d, int levels) {
 
 // a colour-split array of one grid
 static size_t array_bytes(const Grid& g) { return ((size_t)g.m * 8 + 255) & ~(size_t)255; }
+// the workspace: r and v per component and s, of every level
+static size_t fmg_bytes(const std::vector<Dims>& levels, int comps) {
+    size_t b = 0;
+    for (Dims d : levels) b += (2 * comps + 1) * array_bytes(Grid(d));
+    return b + NPART * sizeof(double) + 256;
+}
 
 }  // namespace tsf
 
@@ -702,10 +709,7 @@ extern "C" {
 
 size_t tsf_gvf_fmg_workspace_size(tsf_dims dims, int32_t levels) {
     if (levels < 0 || levels > 12) return 0;
-    const size_t arrays = 2 * (D(dims).n() <= FMG_TOGETHER ? 3 : 1) + 1;  // r and v per component, s
-    size_t b = 0;
-    for (Dims d : level_dims(D(dims), levels)) b += arrays * array_bytes(Grid(d));
-    return b + NPART * sizeof(double) + 256;
+    return fmg_bytes(level_dims(D(dims), levels), D(dims).n() <= FMG_TOGETHER ? 3 : 1);
 }
 
 tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, float mu, int32_t iterations,
@@ -725,13 +729,15 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
     if (f->x == out->x || f->y == out->y || f->z == out->z)
         return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: f and out planes must not alias", W);
     Scratch sc;
-    TSF_TRY(sc.get(workspace, workspace_bytes, tsf_gvf_fmg_workspace_size(dims, levels), W));
+    // a workspace too small for three components runs them one by one
+    const bool together = D(dims).n() <= FMG_TOGETHER && (!workspace || workspace_bytes >= fmg_bytes(ld, 3));
+    TSF_TRY(sc.get(workspace, workspace_bytes, fmg_bytes(ld, together ? 3 : 1), W));
     Solver S;
     S.mu = mu;
     S.v0 = v0;
     S.v1 = v1;
     S.v2 = v2;
-    S.comps = D(dims).n() <= FMG_TOGETHER ? 3 : 1;
+    S.comps = together ? 3 : 1;
     S.st = stream;
     char* p = (char*)sc.ptr;
     for (Dims d : ld) {
