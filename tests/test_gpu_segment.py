@@ -97,6 +97,35 @@ def test_segment_lists_and_dense_passes(tsf, orc, nx, half, step):
     assert passes == opasses and np.array_equal(got, exp)
 
 
+@pytest.mark.parametrize("cells,side", [(1, 15), (1, 16), (4, 15), (4, 16)])
+def test_segment_list_overflow_while_growing(tsf, orc, cells, side):
+    """Seeds that fit the list (a quarter of the volume) and a first pass whose
+    nominations do not: cells**3 basins, each seeded by a cube of 9**3 - 1
+    around its centre, the field pointing there."""
+    n = cells * side
+    ax = (np.arange(n) % side - (side - 1) // 2).astype(np.float32)
+    d = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"))[::-1]  # x, y, z
+    rho = np.sqrt((d * d).sum(0))
+    m = (np.where(rho <= 6, rho, np.maximum(0, 12 - rho)) / 32).astype(np.float32)
+    F = np.zeros((4, n, n, n), np.float32)
+    F[:3] = -m * d / np.where(rho > 0, rho, 1)
+    F[3] = np.where(m > 0, m, 1e-3)
+    cl = (rho == 0).astype(np.uint8)
+    # the voxels that the first pass nominates: not the centre, pointing at a
+    # seed of smaller magnitude
+    cap = (n ** 3 + 255) // 256 * 64
+    seeds = np.abs(d).max(0) <= 4
+    dirs = np.array([(a, b, c) for a in (-1, 0, 1) for b in (-1, 0, 1) for c in (-1, 0, 1) if (a, b, c) != (0, 0, 0)])
+    unit = dirs / np.sqrt((dirs ** 2).sum(1))[:, None]
+    to = dirs[np.tensordot(unit, F[:3], 1).argmax(0)]  # (..., 3): x, y, z
+    at = [np.clip(i + to[..., 2 - k], 0, n - 1) for k, i in enumerate(np.indices(F.shape[1:]))]
+    nominated = (rho > 0) & seeds[tuple(at)] & (cl[tuple(at)] == 0) & (F[3] > F[3][tuple(at)])
+    assert seeds.sum() - cl.sum() <= cap < nominated.sum()
+    got, passes = run_device(tsf, cl, np.full(cl.shape, 8.0, np.float32), F)
+    exp, opasses = orc.segment_inverse_gradient(cl, np.full(cl.shape, 8.0, np.float32), F)
+    assert passes == opasses and np.array_equal(got, exp)
+
+
 @pytest.mark.parametrize("seed", [5, 6])
 def test_segment_direction_ties_vs_oracle(tsf, orc, seed):
     """Fields of small whole numbers: equal and zero components, zero vectors

@@ -235,13 +235,18 @@ template <class S>
 __global__ void __launch_bounds__(256) k_seg_grow_list(const uint8_t* __restrict__ cur, Field<S> F, Dims d,
                                                        const int32_t* __restrict__ list, int32_t* __restrict__ next,
                                                        int cap, uint8_t* marks, SegSlots* s, int p, bool first) {
-    if (seg_skip(s, p, first)) return;
     __shared__ int32_t own[GROW_OWN];
-    __shared__ int found, grown;
+    __shared__ int found, grown, skip;
+    // One verdict for the workgroup: another one's append may set the overflow
+    // mark at any time, and waves that read it apart would part ways here.
+    if (threadIdx.x == 0) {
+        skip = seg_skip(s, p, first);
+        found = grown = 0;
+    }
+    __syncthreads();
+    if (skip) return;
     const unsigned accepted = (p & 1) ? 4u : 1u, nominated = 2 * accepted;
     const int count = s->count[p];
-    if (threadIdx.x == 0) found = grown = 0;
-    __syncthreads();
     const int sub = threadIdx.x & 31;
     const int a = sub / 9 - 1, b = sub / 3 % 3 - 1, c = sub % 3 - 1;
     for (int k0 = blockIdx.x * 8; k0 < count; k0 += gridDim.x * 8) {
