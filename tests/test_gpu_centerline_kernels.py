@@ -31,6 +31,37 @@ def test_nms_reach(tsf, orc, cap):
     assert np.array_equal(out.download(), orc.candidate_nms(tdf, rad, V, pos, cap, "f32"))
 
 
+@pytest.mark.parametrize("axis", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 0), (1, 0, 1), (0, 1, 1), (1, -1, 0)])
+def test_nms_straight_tubes(tsf, orc, axis):
+    """Offsets in the plane across the tube and along its axis, where the
+    cosine of their angle to the plane rounds to more than 1 (its arc cosine
+    is NaN and the offset does not count) or is made of rounding errors.  A
+    cell of 15^3 for each: a candidate in its middle and one darker voxel."""
+    e = np.array(axis) / np.linalg.norm(axis)
+    k = np.arange(-7, 8)
+    r = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3)  # x, y, z
+    r2 = (r * r).sum(1)
+    along = (r @ e) ** 2
+    r = r[(r2 > 0) & (r2 < 64) & ((along <= 0.02 * r2) | (along >= 0.98 * r2))]
+    m = int(np.ceil(len(r) ** (1 / 3)))
+    n = 15 * m
+    c = np.indices((n, n, n))[::-1] % 15 - 7.0  # x, y, z from the middle of the cell
+    F = np.ones((4, n, n, n), np.float32)
+    F[:3] = -(c - e[:, None, None, None] * np.tensordot(e, c, 1)) / 20
+    cell = np.stack(np.unravel_index(np.arange(len(r)), (m, m, m)), 1)[:, ::-1]
+    pos = np.ascontiguousarray(15 * cell + 7, np.int32)
+    F[3][tuple((pos + r).T[::-1])] = 0.5
+    rad = np.full((n, n, n), 8, np.float32)
+    out = tsf.DeviceArray((n, n, n), np.uint8)
+    out.zero()
+    tsf.candidate_nms(_dev(tsf, rad), _dev(tsf, rad), tsf.Field.from_host(F), _dev(tsf, pos), len(pos), 8, out)
+    exp = orc.candidate_nms(rad, rad, F, pos, 8, "f32")
+    across = (r @ e) ** 2 < 1e-6
+    kept = exp[tuple(pos.T[::-1])][across]
+    assert 0 < kept.sum() < len(kept)
+    assert np.array_equal(out.download(), exp)
+
+
 @pytest.mark.parametrize("shape", [(9, 11, 516), (10, 7, 131), (5, 5, 8), (65, 66, 68)])
 @pytest.mark.parametrize("cube", [1, 4, 5, 7, 64])
 def test_cube_max_rows(tsf, orc, shape, cube):

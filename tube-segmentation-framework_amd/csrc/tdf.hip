@@ -69,34 +69,40 @@ __global__ void k_do_eigen_points(const float* __restrict__ Fx, const float* __r
 //
 // The angle test of the reference, theta = acos(r/|r| . p/|p|) with p = r -
 // e1 (e1 . r), is sin^2 of the angle between r and that plane: for a unit e1
-// theta < 0.5 exactly when (e1 . r)^2 < sin^2(0.5) |r|^2.  Offsets clear of
-// that bound by 1e-4 |r|^2 (the float expressions are within 1e-5 of it) are
+// theta < 0.5 where (e1 . r)^2 < sin^2(0.5) |r|^2.  Offsets clear of that
+// bound by 1e-4 |r|^2 (the float expressions are within 1e-5 of it) are
 // decided by it; the others, and all of them when e1 is not of unit length to
-// 1e-5, by the reference's own expressions.
+// 1e-5, by the reference's own expressions.  So are the two ends:
+//   - r in the plane: the cosine may round to more than 1, its acos is NaN and
+//     the offset does not count (36 of the 192 offsets across an axis-aligned
+//     tube with |r| < 8).  Its rounding error is below 6e-7 (ten roundings), its
+//     distance from 1 half of (e1 . r)^2 / |r|^2;
+//   - r along e1: p is what rounding leaves and may point anywhere.
+// (Evaluated for 1326 axes and all offsets up to 63, the expressions differ from
+// the bound at and below 2.0e-7 and at and above 0.99999 of |r|^2 only.)  They
+// are asked about darker voxels alone, of which a survivor has few.
 struct NmsCandidate {
     int x, y, z, maxD;
     float ex, ey, ez, wp;
     bool unit;
 };
-__device__ __forceinline__ bool nms_in_plane(const NmsCandidate& q, int a, int b, int c) {
+template <class S>
+__device__ __forceinline__ bool nms_beaten(const NmsCandidate& q, const Field<S>& F, const Dims& d, int a, int b,
+                                           int c) {
+    const int n2 = a * a + b * b + c * c;
+    if (n2 == 0 || n2 >= q.maxD * q.maxD) return false;
     const float rx = (float)a, ry = (float)b, rz = (float)c;
     const float dp = q.ex * rx + q.ey * ry + q.ez * rz;
-    const float r2 = (float)(a * a + b * b + c * c), d2 = dp * dp;
-    if (q.unit && d2 < 0.2297488f * r2) return true;
-    if (q.unit && d2 > 0.2299488f * r2) return false;
+    const float r2 = (float)n2, d2 = dp * dp;
+    if (q.unit && d2 > 0.2299488f * r2 && d2 < 0.999f * r2) return false;
+    const int nx = clampi(q.x + a, 0, d.X - 1), ny = clampi(q.y + b, 0, d.Y - 1), nz = clampi(q.z + c, 0, d.Z - 1);
+    if (!(F.mag(d.at(nx, ny, nz)) < q.wp)) return false;
+    if (q.unit && d2 < 0.2297488f * r2 && d2 > 4e-6f * r2) return true;
     const float px = rx - q.ex * dp, py = ry - q.ey * dp, pz = rz - q.ez * dp;
     const float lr = sqrtf(rx * rx + ry * ry + rz * rz);
     const float lp = sqrtf(px * px + py * py + pz * pz);
     const float cs = (rx / lr) * (px / lp) + (ry / lr) * (py / lp) + (rz / lr) * (pz / lp);
     return acosf(cs) < 0.5f;
-}
-template <class S>
-__device__ __forceinline__ bool nms_beaten(const NmsCandidate& q, const Field<S>& F, const Dims& d, int a, int b,
-                                           int c) {
-    const int r2 = a * a + b * b + c * c;
-    if (r2 == 0 || r2 >= q.maxD * q.maxD || !nms_in_plane(q, a, b, c)) return false;
-    const int nx = clampi(q.x + a, 0, d.X - 1), ny = clampi(q.y + b, 0, d.Y - 1), nz = clampi(q.z + c, 0, d.Z - 1);
-    return F.mag(d.at(nx, ny, nz)) < q.wp;
 }
 // A thread solves for its candidate's e1 and looks at the 26 voxels next to
 // it, which rejects most candidates off the axis; the survivors with a wider
