@@ -82,6 +82,18 @@ def test_workspace_sizes():
     assert tsf.gvf_fmg_workspace_size((64, 64, 64), 2) > 5 * 64 ** 3 * 4
 
 
+@pytest.mark.parametrize("shape,sums", [((64, 64, 64), 28), ((48, 60, 200), 48), ((128, 128, 128), 156),
+                                        ((512, 512, 512), 7488), ((4, 4, 4), 2), ((248, 670, 17), 536)])
+def test_gvf_adjoint_workspace_size_follows_from_the_arguments(shape, sums):
+    """States, folded adjoints and a fixed number of double sums: the same
+    with and without a device, and what callers have allocated before."""
+    import tsf
+    for every in (1, 7, 50):
+        floats = (every + 2) * 3 * int(np.prod(shape)) * 4
+        need = (floats + 255) // 256 * 256 + (1024 + 1 + sums) * 8
+        assert tsf.gvf_euler_adjoint_workspace_size(shape, every) == need
+
+
 def test_hp_compact_noalloc_rejects_extent_above_scratch():
     """The no-allocation compaction refuses volumes whose largest extent
     exceeds its static scratch (1024) on the host, before any device work."""

@@ -116,6 +116,34 @@ def test_gvf_adjoint_recompute_bit_exact(tsf, sh):
         assert abs(dmu - out[0][1]) <= 1e-12 * abs(out[0][1])
 
 
+@pytest.mark.parametrize("sh,sums", [((64, 64, 64), 28), ((48, 60, 200), 48), ((248, 670, 17), 536)])
+def test_gvf_adjoint_in_its_workspace(tsf, sh, sums):
+    """Small volumes in many chunks and a thin one whose chunks are lengthened:
+    several reverse steps per launch in a workspace of the size that the
+    extents give, nothing written behind it, the gradients of single steps."""
+    iters, mu, every = 5, 0.07, 5
+    g = rng(8)
+    F = np.zeros((4,) + sh, np.float32)
+    F[:3] = g.uniform(-1, 1, (3,) + sh) / np.sqrt(3)
+    F[3] = 1
+    dV = tsf.DeviceArray.from_host(g.standard_normal((3,) + sh).astype(np.float32))
+    f = tsf.Field.from_host(F)
+    need = ((every + 2) * 3 * int(np.prod(sh)) * 4 + 255) // 256 * 256 + (1025 + sums) * 8
+    ws = tsf.DeviceArray.from_host(np.full(need + 4096, 0xa5, np.uint8))
+    ws.nbytes = need
+    out = []
+    for k, w in ((1, None), (every, ws)):
+        cps = tsf.DeviceArray((tsf.gvf_checkpoint_count(iters, k), 3) + sh, np.float32)
+        tsf.gvf_euler_checkpointed(f, tsf.Field(sh), mu, iters, k, cps)
+        dF = tsf.DeviceArray((3,) + sh, np.float32)
+        dmu = tsf.gvf_euler_adjoint(f, mu, iters, k, cps, dV, dF, w)
+        out.append((dF.download(), dmu))
+    ws.nbytes += 4096
+    assert np.all(ws.download()[need:] == 0xa5)
+    assert np.array_equal(out[0][0], out[1][0])
+    assert abs(out[0][1] - out[1][1]) <= 1e-12 * abs(out[0][1])
+
+
 def test_gvf_finish_adjoint(tsf):
     g = rng(7)
     sh = (6, 7, 8)

@@ -406,15 +406,6 @@ __global__ void __launch_bounds__(ABX* ABY, 4) k_gvf_adj_march(P3 Lf, P3 v, P3 F
     if (tid == 0) part[blockIdx.x + (i64)gridDim.x * (blockIdx.y + (i64)gridDim.y * blockIdx.z)] += sh[0];
 }
 
-// part2[b] = sum of a contiguous chunk of n partials (fixed order)
-__global__ void __launch_bounds__(RB) k_reduce_parts(const double* __restrict__ part, i64 n, double* __restrict__ part2) {
-    const i64 chunk = (n + gridDim.x - 1) / gridDim.x;
-    const i64 lo = blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
-    double s = 0.0;
-    for (i64 j = lo + threadIdx.x; j < hi; j += RB) s += part[j];
-    block_sum_double(s, &part2[blockIdx.x]);
-}
-
 // W = |V| (1 where |V| == 0): dV += dW V / |V|
 __global__ void k_finish_adjoint(const float* __restrict__ vx, const float* __restrict__ vy,
                                  const float* __restrict__ vz, const float* __restrict__ dW, float* __restrict__ dx,
@@ -802,20 +793,21 @@ static size_t adj_blocks(const Dims& d) {
 // rows are halo.
 enum { ADJ_K2, ADJ_K3, ADJ_FORMS };
 static const ColsForm ADJ[ADJ_FORMS] = {{2, 1, 8, 2, 1.16f, 2.2f}, {3, 1, 12, 1, 1.85f, 1.85f}};
+// d/dmu sums, one per block of the marching kernels and added up over launches.
+// Their number is part of the workspace's size, so it follows from the extents
+// alone: NPART, and the blocks of k_gvf_adj_march or of two sets on tiles of
+// 60 x 10 columns and 64 planes, whichever are more.  k_gvf_adj_cols takes no
+// more blocks than that, which lengthens the chunks of thin volumes only (248 x
+// 670 x 17: 1560 blocks where its own choice is 2016).
+static size_t adj_sums(const Dims& d) {
+    const size_t pairs = 2 * (size_t)((d.X + 59) / 60) * ((d.Y + 9) / 10) * ((d.Z + 63) / 64);
+    return NPART + std::max(adj_blocks(d), pairs);
+}
 static ColsPlan adj_plan(int form, const Dims& d) {
     const ColsForm& c = ADJ[form];
     // the adjoint and f with the planes beside the chunk; the states, dF read
     // and written, the adjoint written
-    return cols_plan(c, form, d, d.Z, 0.0, 24.0, 36.0 + 12.0 * c.K);
-}
-static size_t adj_cols_blocks(const ColsPlan& p, const Dims& d) {
-    const dim3 g = cols_grid(ADJ[p.form], d, d.Z, p.zc);
-    return (size_t)g.x * g.y * g.z;
-}
-// d/dmu sums: one per block of the marching kernels, added up over launches
-static size_t adj_parts(const Dims& d) {
-    return std::max(adj_blocks(d), std::max(adj_cols_blocks(adj_plan(ADJ_K2, d), d),
-                                            adj_cols_blocks(adj_plan(ADJ_K3, d), d)));
+    return cols_plan(c, form, d, d.Z, 0.0, 24.0, 36.0 + 12.0 * c.K, (double)adj_sums(d));
 }
 
 template <int K, int NW, int WPE>
@@ -983,7 +975,7 @@ static size_t adj_float_bytes(const Dims& d, int k) {
 size_t tsf_gvf_euler_adjoint_workspace_size(tsf_dims dims, int32_t checkpoint_every) {
     const Dims d = D(dims);
     if (checkpoint_every < 1) return 0;
-    return adj_float_bytes(d, checkpoint_every) + (NPART + 1 + adj_parts(d)) * sizeof(double);
+    return adj_float_bytes(d, checkpoint_every) + (1 + adj_sums(d)) * sizeof(double);
 }
 
 tsf_status tsf_gvf_euler_adjoint(const tsf_field* f, tsf_dims dims, float mu, int32_t iterations,
@@ -1005,14 +997,13 @@ tsf_status tsf_gvf_euler_adjoint(const tsf_field* f, tsf_dims dims, float mu, in
     float* seg = (float*)sc.ptr;              // k states of 3 planes
     float* lamA = seg + (i64)k * 3 * N;       // folded adjoint, ping-pong
     float* lamB = lamA + 3 * N;
-    double* part2 = (double*)((char*)sc.ptr + adj_float_bytes(d, k));  // NPART
-    double* acc = part2 + NPART;
-    double* part = acc + 1;                   // one per stencil block
-    const i64 nparts = (i64)adj_parts(d);
+    double* acc = (double*)((char*)sc.ptr + adj_float_bytes(d, k));
+    double* part = acc + 1;                   // one per block
+    const int nparts = (int)adj_sums(d);
+    const ColsPlan two = adj_plan(ADJ_K2, d), three = adj_plan(ADJ_K3, d);
     // several reverse steps per launch address three volumes with 32-bit
     // byte offsets
-    const bool cols = 3 * N * (i64)sizeof(float) < ((i64)1 << 31);
-    const ColsPlan two = adj_plan(ADJ_K2, d), three = adj_plan(ADJ_K3, d);
+    const bool cols = 3 * N * (i64)sizeof(float) < ((i64)1 << 31) && two.us < 1e30f && three.us < 1e30f;
     const bool prefer_two = two.us * 3 < three.us * 2;
     const float* fp[3] = {(const float*)f->x, (const float*)f->y, (const float*)f->z};
     hipError_t e = hipMemsetAsync(dF, 0, 3 * N * sizeof(float), stream);
@@ -1068,8 +1059,7 @@ tsf_status tsf_gvf_euler_adjoint(const tsf_field* f, tsf_dims dims, float mu, in
             n -= k;
         }
     }
-    hipLaunchKernelGGL(k_reduce_parts, NPART, RB, 0, stream, part, nparts, part2);
-    hipLaunchKernelGGL(k_fold_partials, 1, RB, 0, stream, part2, NPART, acc);
+    hipLaunchKernelGGL(k_fold_partials, 1, RB, 0, stream, part, nparts, acc);
     TSF_TRY(check_launch(W));
     double h = 0.0;
     TSF_TRY(sync_read_double(acc, &h, stream, W));

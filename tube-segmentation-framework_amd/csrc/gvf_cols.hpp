@@ -558,19 +558,21 @@ inline dim3 cols_grid(const ColsForm& c, Dims d, int planes, int zc) {
 // last round part full; a launch also moves `once` bytes a voxel and `halo`
 // bytes that the planes beside a chunk repeat, and costs about 5 us to start
 // and to fill the pipeline.  range: bytes per plane that a chunk's buffer
-// resources cover (0: no limit from them).
+// resources cover (0: no limit from them).  max_blocks: workgroups that a
+// launch may have.  us stays 1e30 where nothing fits.
 struct ColsPlan {
     int form, zc;
     float us;
 };
-inline ColsPlan cols_plan(const ColsForm& c, int form, Dims d, int planes, double range, double halo, double once) {
+inline ColsPlan cols_plan(const ColsForm& c, int form, Dims d, int planes, double range, double halo, double once,
+                          double max_blocks = 1e30) {
     const double cus = cu_count();
     ColsPlan best{form, 2, 1e30f};
     for (int steps = (2 * c.K + 3) & ~3; steps <= 140; steps += 4) {
         const int zc = steps - 2 * (c.K - 1);
         if (zc < 2 || range * (steps + 4) >= 2147483648.0) continue;
         const dim3 g = cols_grid(c, d, planes, zc);
-        const double per_cu = (double)g.x * g.y * g.z / cus;
+        const double blocks = (double)g.x * g.y * g.z, per_cu = blocks / cus;
         double t;
         if (per_cu <= c.occ) {
             const double n = ceil(per_cu);
@@ -582,7 +584,7 @@ inline ColsPlan cols_plan(const ColsForm& c, int form, Dims d, int planes, doubl
         }
         const double memory = (double)d.n() * (halo * (zc + 2 * c.K) / zc + once) / 4.0e6;  // 4 TB/s
         const float us = (float)fmax(t * steps, memory) + 5.0f;
-        if (us < best.us) best = ColsPlan{form, zc, us};
+        if (us < best.us && blocks <= max_blocks) best = ColsPlan{form, zc, us};
         if (zc >= planes) break;
     }
     return best;
