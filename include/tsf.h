@@ -255,7 +255,9 @@ size_t tsf_gvf_euler_sr_workspace_size(tsf_dims dims, int32_t f32_tail);
  * w = |v| (no zero guard, MGGVFFinish 2202-2216).  F32 storage only.
  * `residual_norms` (optional, host array of 3*iterations doubles) receives
  * the L2 norm of each component's residual before every correction, reduced
- * in double on the device. */
+ * in double on the device.  Workspace: tsf_gvf_fmg_workspace_size; one of five
+ * F32 arrays per grid is enough too (the components then run one by one, in
+ * memory of the call's own where rows of 4 or 9 elements need more). */
 tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, float mu, int32_t iterations,
                        int32_t levels, int32_t v0, int32_t v1, int32_t v2, double* residual_norms,
                        void* workspace, size_t workspace_bytes, hipStream_t stream);

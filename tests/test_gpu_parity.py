@@ -303,6 +303,31 @@ def test_gvf_fmg_small_workspace(tsf, orc):
         tsf.gvf_fmg(f, out, 0.15, 2, levels, workspace=tsf.DeviceArray((n // 2,), np.uint8))
 
 
+@pytest.mark.parametrize("shape,levels", [((20, 18, 4), 0), ((11, 40, 9), 0), ((5, 5, 5), 1), ((10, 6, 4), 1),
+                                          ((4, 4, 4), 0), ((16, 16, 16), 2)])
+def test_gvf_fmg_workspace_of_five_grids(tsf, orc, shape, levels):
+    # five plain arrays of every level hold one component's padded ones but
+    # for rows of 4 or 9 elements and the smallest volumes; a byte less than
+    # both is refused
+    F = _field_from(orc, phantom(shape, 11), fmax=0.2)
+    five, one, dims = 8192 + 256, 8192 + 256, shape
+    for _ in range(levels + 1):
+        five += 5 * ((4 * int(np.prod(dims)) + 255) // 256 * 256)
+        xs = ((dims[2] + 1) // 2 + 3) // 4 * 4
+        one += 3 * ((8 * xs * dims[0] * dims[1] + 255) // 256 * 256)
+        dims = ((1 << (max(dims) - 1).bit_length()) // 2,) * 3
+    out = tsf.Field(shape)
+    ws = tsf.DeviceArray.from_host(np.full(five + 4096, 0xa5, np.uint8))
+    ws.nbytes = five
+    tsf.gvf_fmg(tsf.Field.from_host(F), out, 0.15, 2, levels, workspace=ws)
+    assert np.array_equal(out.download(), orc.gvf_fmg(F, 0.15, 2, 1, 2, 2, levels, "f32"))
+    ws.nbytes = five + 4096
+    assert np.all(ws.download()[five:] == 0xa5)
+    ws.nbytes = min(five, one) - 1
+    with pytest.raises(tsf.TSFError):
+        tsf.gvf_fmg(tsf.Field.from_host(F), out, 0.15, 2, levels, workspace=ws)
+
+
 def test_gvf_fmg_one_component_at_a_time(tsf):
     """Above 2^27 cells the components share one set of buffers: what one
     leaves there must not reach the next, so permuted components (with a zero

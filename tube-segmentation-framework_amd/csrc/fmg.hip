@@ -35,6 +35,8 @@
 // half-sweeps 24-28 us for 134 MB; two of them to a launch would have to read
 // the halo of both).
 #include <math.h>
+
+#include <algorithm>
 #include <vector>
 
 #include "tsf_common.hpp"
@@ -700,6 +702,14 @@ static size_t fmg_bytes(const std::vector<Dims>& levels, int comps) {
     for (Dims d : levels) b += (2 * comps + 1) * array_bytes(Grid(d));
     return b + NPART * sizeof(double) + 256;
 }
+// five plain arrays of every level: what callers were told while the grids
+// were whole, more than one component needs but for rows of 4 or 9 elements
+// (their padding) and a few smallest volumes (the arrays' alignment)
+static size_t five_grids_bytes(const std::vector<Dims>& levels) {
+    size_t b = 0;
+    for (Dims d : levels) b += 5 * (((size_t)d.n() * 4 + 255) & ~(size_t)255);
+    return b + NPART * sizeof(double) + 256;
+}
 
 }  // namespace tsf
 
@@ -729,9 +739,12 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
     if (f->x == out->x || f->y == out->y || f->z == out->z)
         return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: f and out planes must not alias", W);
     Scratch sc;
-    // a workspace too small for three components runs them one by one
+    // a workspace too small for three components runs them one by one; one of
+    // five plain arrays too small even for that is accepted and not used
     const bool together = D(dims).n() <= FMG_TOGETHER && (!workspace || workspace_bytes >= fmg_bytes(ld, 3));
-    TSF_TRY(sc.get(workspace, workspace_bytes, fmg_bytes(ld, together ? 3 : 1), W));
+    const size_t need = fmg_bytes(ld, together ? 3 : 1), five = five_grids_bytes(ld);
+    TSF_TRY(sc.get(workspace, workspace_bytes, workspace ? std::min(need, five) : need, W));
+    if (workspace && workspace_bytes < need) TSF_TRY(sc.get(nullptr, 0, need, W));
     Solver S;
     S.mu = mu;
     S.v0 = v0;
