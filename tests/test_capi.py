@@ -82,6 +82,21 @@ def test_workspace_sizes():
     assert tsf.gvf_fmg_workspace_size((64, 64, 64), 2) > 5 * 64 ** 3 * 4
 
 
+def test_gvf_fmg_asks_for_less_when_memory_is_short():
+    """Without a workspace the multigrid solver asks for three components'
+    arrays and, refused, for one's (here there is no device to give either)."""
+    import tsf
+    if tsf.device_count() > 0:
+        pytest.skip("a device would give the memory")
+    L = tsf.lib()
+    f, out = tsf.FieldDesc(4, 8, 12, 16, 0, 1.0), tsf.FieldDesc(20, 24, 28, 32, 0, 1.0)
+    st = L.tsf_gvf_fmg(ctypes.byref(f), ctypes.byref(out), tsf.Dims(64, 64, 64), 0.1, 1, 2, 1, 2, 2, None, None, 0,
+                       None)
+    one = 3 * 4 * (64 ** 3 + 32 ** 3 * (1 + 1 / 8)) + 8192 + 256
+    assert one < tsf.gvf_fmg_workspace_size((64, 64, 64), 2)
+    assert st == 4 and b"hipMalloc(%d)" % one in L.tsf_last_error()
+
+
 @pytest.mark.parametrize("shape,sums", [((64, 64, 64), 28), ((48, 60, 200), 48), ((128, 128, 128), 156),
                                         ((512, 512, 512), 7488), ((4, 4, 4), 2), ((248, 670, 17), 536)])
 def test_gvf_adjoint_workspace_size_follows_from_the_arguments(shape, sums):

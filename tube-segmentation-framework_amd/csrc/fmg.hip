@@ -739,12 +739,19 @@ tsf_status tsf_gvf_fmg(const tsf_field* f, const tsf_field* out, tsf_dims dims, 
     if (f->x == out->x || f->y == out->y || f->z == out->z)
         return set_error(TSF_ERR_INVALID_ARGUMENT, "%s: f and out planes must not alias", W);
     Scratch sc;
-    // a workspace too small for three components runs them one by one; one of
-    // five plain arrays too small even for that is accepted and not used
-    const bool together = D(dims).n() <= FMG_TOGETHER && (!workspace || workspace_bytes >= fmg_bytes(ld, 3));
-    const size_t need = fmg_bytes(ld, together ? 3 : 1), five = five_grids_bytes(ld);
-    TSF_TRY(sc.get(workspace, workspace_bytes, workspace ? std::min(need, five) : need, W));
-    if (workspace && workspace_bytes < need) TSF_TRY(sc.get(nullptr, 0, need, W));
+    // a workspace, or a device, short of three components' arrays runs them one
+    // by one; a workspace of five plain arrays too small even for that is
+    // accepted and not used
+    const size_t one = fmg_bytes(ld, 1), three = fmg_bytes(ld, 3);
+    bool together = D(dims).n() <= FMG_TOGETHER;
+    if (workspace) {
+        together = together && workspace_bytes >= three;
+        TSF_TRY(sc.get(workspace, workspace_bytes, std::min(one, five_grids_bytes(ld)), W));
+        if (workspace_bytes < one) TSF_TRY(sc.get(nullptr, 0, one, W));
+    } else {
+        together = together && sc.get(nullptr, 0, three, W) == TSF_OK;
+        if (!together) TSF_TRY(sc.get(nullptr, 0, one, W));
+    }
     Solver S;
     S.mu = mu;
     S.v0 = v0;

@@ -85,6 +85,7 @@ tsf_status Scratch::get(void* ws, size_t ws_bytes, size_t need, const char* what
     hipError_t e = hipMalloc(&ptr, need);
     if (e != hipSuccess) {
         ptr = nullptr;
+        (void)hipGetLastError();  // reported here; the caller may go on with less
         return set_error(TSF_ERR_OUT_OF_MEMORY, "%s: hipMalloc(%zu) failed: %s", what, need, hipGetErrorString(e));
     }
     owned = true;
