@@ -280,8 +280,9 @@ static float storage_unit(float scale) {
     return std::is_same<S, SN16>::value ? 32768.0f : scale;
 }
 
-// Whether the multi-step kernel can run: f and v in the same units, and the
-// bytes of a chunk's planes addressable by a buffer resource.
+// Whether the multi-step kernel can run: f and v in the same units, and 73
+// planes (77 for launches of four) within the 2^31 bytes of a buffer resource,
+// which is more than the shortest chunks need.  Wider planes take single steps.
 template <class S>
 static bool cols_ok(float scale_f, float scale_v, Dims d, int steps) {
     const double span = (double)d.X * d.Y * sizeof(typename S::T) * (64 + (steps == 4 ? 13 : 9));
@@ -291,13 +292,14 @@ static bool cols_ok(float scale_f, float scale_v, Dims d, int steps) {
 // The built forms of k_gvf_cols.  Small tiles keep a small volume's steps
 // short and its workgroups many; four steps per launch save HBM traffic, and
 // three rows per thread the tile's overlap, where a volume fills the chip.
+// {}: not built for the storage.
 enum { K2_SMALL, K2_TALL, K2_ROWS2, K3, K4_TALL, K4_ROWS3, COLS_FORMS };
 static const ColsForm FORMS_F32[COLS_FORMS] = {
-    {2, 1, 8, 3, 0.80f, 1.50f}, {2, 1, 16, 1, 1.12f, 1.12f}, {2, 2, 8, 2, 1.33f, 2.1f},
+    {2, 1, 8, 3, 0.80f, 1.50f}, {2, 1, 16, 1, 1.12f, 1.12f}, {},
     {3, 1, 16, 1, 1.45f, 1.45f}, {4, 1, 16, 1, 1.70f, 1.70f}, {4, 3, 8, 1, 2.75f, 2.75f}};
 static const ColsForm FORMS_16[COLS_FORMS] = {
-    {2, 1, 8, 3, 1.00f, 1.66f}, {2, 1, 16, 1, 1.40f, 1.40f}, {2, 2, 8, 2, 1.67f, 2.35f},
-    {3, 1, 16, 1, 2.10f, 2.10f}, {4, 1, 16, 1, 2.90f, 2.90f}, {4, 3, 8, 1, 4.5f, 4.5f}};
+    {2, 1, 8, 3, 1.00f, 1.66f}, {}, {2, 2, 8, 2, 1.67f, 2.35f},
+    {}, {4, 1, 16, 1, 2.90f, 2.90f}, {}};
 
 template <class S>
 static const ColsForm* cols_forms() {
@@ -378,14 +380,9 @@ static StepsF32 steps_f32(int iters, Dims d, bool ok, bool mids) {
     const int K = FORMS_F32[s.main.form].K;
     s.mains = iters / K;
     int r = iters % K;
-    if (r == 1) {
-        if (s.mains == 0) {
-            s.ones = 1;
-            r = 0;
-        } else {
-            s.mains--;
-            r += K;
-        }
+    if (r == 1) {  // mains >= 1, since iters >= 2
+        s.mains--;
+        r += K;
     }
     s.threes = r & 1;
     s.twos = (r - 3 * s.threes) / 2;

@@ -161,9 +161,7 @@ struct Cols {
     const ColsArgs<S>& a;
     Lds* L;
     int lane, w, row0, qs, qe, zb;
-    // 0 or 1, uniform; one word each, as the test of a bit of a common word is
-    // miscompiled below (the branch inverted where the test is reused)
-    int ledge, redge, yfix, yface;
+    int ledge, redge, yfix, yface;  // 0 or 1, uniform
     bool col0, colN;
     unsigned pb, rb, voff, hoff;
     unsigned svoff[R];  // store offset of the thread's lane, NO_LANE on rows it does not store
@@ -328,7 +326,6 @@ struct Cols {
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int p = t - k;
-            
             if (k > 0 && zedge) {
                 if (p == 1)
 #pragma unroll
