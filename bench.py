@@ -204,7 +204,8 @@ def main():
     gvox = N * args.iters / (gvf_ms * 1e-3) / 1e9
 
     # the dominant kernel's average launch: two GVF runs that differ only in
-    # K launches of it (each followed by its small face-copy kernel)
+    # K launches of it (the precision form's each followed by its small
+    # face-copy kernel)
     def gvf_time(iters, reps=3):
         ts = []
         for _ in range(reps):
@@ -223,12 +224,16 @@ def main():
                  "bf16": "k_gvf_sr2<BF16, BF16, BF16, false>"}[args.storage]
         bytes_per_voxel = 18  # v and f read, v written: 3 components x 2 bytes each
     else:
-        # F32 runs group iterations as is fastest (four a launch at this size)
-        spl = 4 if args.storage == "f32" and args.fuse >= 2 else args.fuse
+        # with fuse >= 2, SNORM16 goes in pairs and F32 as is fastest: four a
+        # launch at 512^3, elsewhere perhaps other launches for the four
+        # iterations that are timed
+        spl = {"f32": 4, "sn16": 2}.get(args.storage, args.fuse) if args.fuse >= 2 else 1
         K = 48 // spl
         launch_ms = (gvf_time(spl * (K + 2)) - gvf_time(2 * spl)) / K
         gk = {4: "k_gvf_cols<{}, 4>", 2: "k_gvf_cols<{}, 2>"}.get(spl, "k_gvf_march<{}, 2, false>")
         kname = gk.format(args.storage.upper())
+        if args.storage == "f32" and args.fuse >= 2 and n != 512:
+            kname = "k_gvf_cols<F32>, four iterations"
         bytes_per_voxel = 9 * (4 if S == tsf.STORAGE_F32 else 2)
     achieved = bytes_per_voxel * N / (launch_ms * 1e-3)
 
@@ -238,8 +243,8 @@ def main():
     if not args.no_downstream:
         downstream = downstream_stages(vol, shape, t_s, r_s, V, stream)
 
-    # the same forward in FP32: four GVF steps per launch (the fastest FP32
-    # form) and one (the plain FP32 path)
+    # the same forward in FP32: several GVF steps per launch (the fastest FP32
+    # form, four at 512^3) and one (the plain FP32 path)
     f32 = None
     if not args.no_f32_compare and not (S == tsf.STORAGE_F32 and not precision):
         Fs32, F32, V32 = tsf.Field(shape), tsf.Field(shape), tsf.Field(shape)
