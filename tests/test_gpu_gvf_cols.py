@@ -34,7 +34,10 @@ def test_tile_edges(tsf, shape, iters, storage):
     _both(tsf, shape, iters, storage)
 
 
-@pytest.mark.parametrize("shape,iters,storage", [((200, 401, 301), 7, F32), ((150, 300, 290), 5, SN16)])
+@pytest.mark.parametrize("shape,iters,storage", [
+    ((200, 401, 301), 7, F32), ((150, 300, 290), 5, SN16),
+    # few planes, narrow rows, both: within the last-level cache
+    ((11, 310, 290), 9, F32), ((260, 250, 16), 7, F32), ((30, 1300, 31), 6, F32)])
 def test_large_volume(tsf, shape, iters, storage):
     _both(tsf, shape, iters, storage)
 

@@ -310,9 +310,27 @@ template <class S>
 static ColsPlan cols_best(std::initializer_list<int> forms, Dims d) {
     const ColsForm* F = cols_forms<S>();
     constexpr size_t e = sizeof(typename S::T);  // v and f read, the result written
+    constexpr bool f32 = std::is_same<S, F32>::value;
+    // Thin F32 volumes (us an iteration, against the estimate without these
+    // three rules):
+    //   - nine planes beyond the L2s and within the last-level cache come at
+    //     about 8 TB/s (6 x 1000 x 1000: 34.2 in fours, 25.5 in pairs);
+    //   - with few planes the tall tiles then take 1.3 times their step or more
+    //     (6 x 700 x 700: 20.4 on them, 14.4 on small ones; within the L2s they
+    //     stay the better ones: 20 x 128 x 128 5.2 against 6.0);
+    //   - on rows below half a tile's width the small tiles of a full CU step in
+    //     1.33 us (512 x 512 x 8: 48.6 in fours, 42.9 in pairs).
+    // Others are left to the estimate: at 160^3 it chooses 17.6, with the first
+    // rule 18.7.
+    const double bytes = 9.0 * e * d.n();
+    const bool cached = f32 && (d.X < 32 || d.Z < 32) && bytes > 32e6 && bytes <= 235e6;
+    const double m = cached ? 0.5 * e : 1.0 * e;
     ColsPlan best{0, 0, 1e30f};
     for (int f : forms) {
-        const ColsPlan p = cols_plan(F[f], f, d, d.Z - 2, (double)d.X * d.Y * e, 6.0 * e, 3.0 * e);
+        ColsForm c = F[f];
+        if (f32 && f == K2_SMALL && d.X < 32) c.full = 1.33f;
+        if (f32 && f == K2_TALL && cached && d.Z < 32) continue;
+        const ColsPlan p = cols_plan(c, f, d, d.Z - 2, (double)d.X * d.Y * e, 6.0 * m, 3.0 * m);
         if (best.zc == 0 || p.us * F[best.form].K < best.us * F[p.form].K) best = p;
     }
     return best;

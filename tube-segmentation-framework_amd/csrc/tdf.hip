@@ -109,7 +109,7 @@ __device__ __forceinline__ bool nms_beaten(const NmsCandidate& q, const Field<S>
 // reach are collected in LDS and a wave searches each of them, 64 offsets at
 // a time.  192298 candidates of tubes up to radius 8 (reach up to 8: 4913
 // offsets): 3267 us with a thread per candidate and the reference's
-// expressions at every offset, 93 us so.
+// expressions at every offset, 89 us so.
 template <class S>
 __global__ void __launch_bounds__(256) k_candidate_nms(const float* __restrict__ radius, Field<S> F, Dims d,
                                                        const int32_t* __restrict__ pos, i64 count, int cap,
