@@ -314,12 +314,12 @@ static ColsPlan cols_best(std::initializer_list<int> forms, Dims d) {
     // Thin F32 volumes (us an iteration, against the estimate without these
     // three rules):
     //   - nine planes beyond the L2s and within the last-level cache come at
-    //     about 8 TB/s (6 x 1000 x 1000: 34.2 in fours, 25.5 in pairs);
+    //     about 8 TB/s (6 x 1000 x 1000: 33.5 in fours, 28.3 in pairs);
     //   - with few planes the tall tiles then take 1.3 times their step or more
-    //     (6 x 700 x 700: 20.4 on them, 14.4 on small ones; within the L2s they
+    //     (6 x 700 x 700: 20.4 on them, 15.8 on small ones; within the L2s they
     //     stay the better ones: 20 x 128 x 128 5.2 against 6.0);
     //   - on rows below half a tile's width the small tiles of a full CU step in
-    //     1.33 us (512 x 512 x 8: 48.6 in fours, 42.9 in pairs).
+    //     1.33 us (512 x 512 x 8: 49.0 in fours, 43.0 in pairs).
     // Others are left to the estimate: at 160^3 it chooses 17.6, with the first
     // rule 18.7.
     const double bytes = 9.0 * e * d.n();
