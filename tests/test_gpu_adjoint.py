@@ -90,11 +90,11 @@ def test_gvf_adjoint_checkpointed(tsf, orc, iters, every, sh):
 def test_gvf_adjoint_recompute_bit_exact(tsf, sh):
     # every state stored (checkpoint every iteration, nothing recomputed,
     # every reverse step a single launch) against segments of 2 and 11
-    # recomputed by four-step launches and single steps and reversed two
-    # steps per launch (the last pair of segment 0 ends at v^0 = f): the
-    # recomputed states are the stored ones and a two-step launch is two
-    # single ones bit for bit, so dF is identical; dmu sums the same terms
-    # in double over other blocks, so it agrees to double rounding
+    # recomputed and reversed several steps per launch (the last launch of
+    # segment 0 ends at v^0 = f): the recomputed states are the stored ones
+    # and a launch of several steps is as many single ones bit for bit, so dF
+    # is identical; dmu sums the same terms in double over other blocks, so it
+    # agrees to double rounding
     g = rng(5)
     F = np.zeros((4,) + sh, np.float32)
     F[:3] = g.uniform(-1, 1, (3,) + sh) / np.sqrt(3)
